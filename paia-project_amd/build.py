@@ -42,7 +42,8 @@ HIP_FLAGS = [
     f"-I{INCLUDE}", f"-I{CSRC}",
 ]
 HIP_SOURCES = ["gemv_runtime.hip", "gemv_bf16.hip", "gemv_fp8.hip", "gemv_int4.hip", "gemv_dequant.hip",
-               "gemv_select.hip", "quantize.hip", "gemv_batch.hip"]
+               "gemv_select.hip", "quantize.hip", "gemv_batch.hip",
+               "gemv_tile.hip"]
 
 
 def _run(cmd, quiet_warn=True):

@@ -23,6 +23,7 @@
 
 #include "gemv_batch.h"
 #include "gemv_kernel.h"
+#include "gemv_tile.h"
 #include "paia_gemv.h"
 
 namespace {
@@ -254,10 +255,34 @@ int pick(int kind, int M, int N, int K)
     return find(t, P, U, W, S, X);
 }
 
+// Where the row-streaming kernel stays ahead of the tile kernel (both measured, us, rows / tile): the tile kernel reads
+// 16 rows per wave and adds 8 waves' partial sums, which few tiles or few activation rows do not repay.
+//   * at most 128 tiles, where a block per tile leaves half the CUs idle: FP8 1000x3584 M = 2 3.22 / 3.86, M = 4 3.76 /
+//     4.12; BF16 M = 4 4.30 / 5.25, M = 7 and 8 even; INT4 M = 2 3.48 / 4.2, M = 3 even;
+//   * up to 1024 tiles of ordinary K, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even), FP8 M = 2
+//     (6144x4096 6.51 / 7.10, 10112x4096 9.19 / 10.09; M = 3 7.54 / 7.23), INT4 M = 2 up to 256 tiles (4096x4096 4.84 / 5.2;
+//     6144x4096 even). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
+//     kernel's.
+bool rows_ahead(int kind, int M, int N, int K)
+{
+    const int ntiles = (N + kTileRows - 1) / kTileRows;
+    const bool mid = K >= 2048 && K <= 8192;
+    if (kind >= 2) return M == 2 && ntiles <= 256 && mid;
+    if (ntiles <= 128) return M <= (kind == 0 ? 7 : 4);
+    return mid && ntiles <= 1024 && M <= (kind == 0 ? 3 : 2);
+}
+
 int batch_impl(int kind, BatchParams p, int variant, void* stream)
 {
     const Table t = table(kind);
-    if (variant < 0) variant = pick(kind, p.M, p.N, p.K);
+    if (variant < 0) {   // the library's choice: the tile kernel, or the table's best where that is ahead or it refuses
+        if (rows_ahead(kind, p.M, p.N, p.K)) variant = pick(kind, p.M, p.N, p.K);
+        if (variant < 0 || t.v[variant].P != 0) {
+            const int rc = launch_tile_picked(kind, p, static_cast<hipStream_t>(stream));
+            if (rc != kTileRefused) return rc;
+            variant = pick(kind, p.M, p.N, p.K);
+        }
+    }
     if (variant < 0 || variant >= t.n) return -1;
     if (!fits(t.v[variant], p.M)) return -2;
     p.S = t.v[variant].S;
