@@ -127,7 +127,9 @@ PAIA_API int paia_gemv_launch_kind(int kind, int N, int K, int variant);
  * M = 1 only and M = 1..16 is its open item (src/README.md:118, swept by paia-bench/configs/shapes.yaml:63-64).
  * x bf16 [M][K] row-major (16-byte aligned), y bf16 [M][N] row-major (2-byte aligned); the weight operands, their
  * alignment and the K rules are those of the M = 1 entry point of the same format. bias bf16 [N] or NULL.
- * kind: 0 BF16, 1 FP8, 2 INT4 reference format, 3 INT4 asymmetric. variant < 0 = paia_gemv_batch_pick_variant's.
+ * kind: 0 BF16, 1 FP8, 2 INT4 reference format, 3 INT4 asymmetric. variant < 0 = the library's choice: at M >= 2 usually
+ * the tile kernel, which has no entry in the tables, else the entry paia_gemv_batch_pick_variant names (the best of the
+ * table: the M = 1 GEMV at M = 1, a row-streaming or matrix-core variant beyond).
  * Knobs: P tiles of 16 rows per wave, U k-blocks of 128 columns in flight per wave, W waves per block, S waves
  * sharing a tile along K, X = 0 x staged in LDS per K-chunk of up to 64 KiB / 1 x loaded with the weights / 2 x
  * staged as for 0 in K-chunks of up to 80 KiB (or the device's per-block LDS if less). P = 0 marks a

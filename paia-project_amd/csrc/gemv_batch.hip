@@ -10,7 +10,8 @@
 // Variant knobs: P tiles of 16 rows per wave, U k-blocks (128 columns) of loads in flight per wave, W waves per block,
 // S waves sharing a tile along K (split-K inside the block), X how x reaches the matrix cores (0 staged in LDS per
 // K-chunk of up to 64 KiB, 1 loaded with the weights, 2 staged as for 0 in chunks of up to 80 KiB, or the device's
-// per-block LDS if less). variant < 0 selects paia_gemv_batch_pick_variant's.
+// per-block LDS if less). variant < 0 is the library's choice: the tile kernel (gemv_tile.h), which has no table entry, or
+// paia_gemv_batch_pick_variant's entry where that is ahead (rows_ahead) or the tile kernel does not take the call.
 //
 // P = 0 marks the row-streaming kernel instead (gemv_rows_kernel: the M = 1 GEMV's weight stream and decode with one
 // accumulator per activation row, for M = 2..6, BF16 and FP8 also 7, 8): then U is its 1-KiB chunks per item, W its waves per
@@ -261,7 +262,8 @@ int pick(int kind, int M, int N, int K)
 //     4.12; BF16 M = 4 4.30 / 5.25, M = 7 and 8 even; INT4 M = 2 3.48 / 4.2, M = 3 even;
 //   * up to 1024 tiles of ordinary K, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even), FP8 M = 2
 //     (6144x4096 6.51 / 7.10, 10112x4096 9.19 / 10.09; M = 3 7.54 / 7.23), INT4 M = 2 up to 256 tiles (4096x4096 4.84 / 5.2;
-//     6144x4096 even). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
+//     6144x4096 even), and the same at any N for K up to 2560 (BF16 33000x2048 M = 2 21.5 / 22.4); and BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 / 29.4, M = 5 29.2 /
+//     30.7). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
 //     kernel's.
 bool rows_ahead(int kind, int M, int N, int K)
 {
@@ -269,7 +271,8 @@ bool rows_ahead(int kind, int M, int N, int K)
     const bool mid = K >= 2048 && K <= 8192;
     if (kind >= 2) return M == 2 && ntiles <= 256 && mid;
     if (ntiles <= 128) return M <= (kind == 0 ? 7 : 4);
-    return mid && ntiles <= 1024 && M <= (kind == 0 ? 3 : 2);
+    if (kind == 0 && K > 8192) return ntiles > 256 && ntiles <= 512 && M <= 5;
+    return mid && (ntiles <= 1024 || K <= 2560) && M <= (kind == 0 ? 3 : 2);
 }
 
 int batch_impl(int kind, BatchParams p, int variant, void* stream)

@@ -24,8 +24,8 @@
 //     as [group][row] words (scale in the upper half, zero point in the low byte): one conflict-free read per tile and
 //     stage, one VALU operation each to unpack.
 //   * INT4 nibbles are decoded exactly: the byte value q in 0..15 read as e4m3 is q 2^-9 (0..7 subnormal, 8..15 in the
-//     first binade), so v_cvt_scalef32_pk_bf16_fp8 at scale 2^9 gives q. No 128 offset to cancel, the same 7 VALU per 8
-//     weights as placing them under a 0x43 byte.
+//     first binade), so v_cvt_scalef32_pk_bf16_fp8 gives q times any power of two. No 128 offset to cancel, the same 7 VALU
+//     per 8 weights as placing them under a 0x43 byte.
 // Rows of D are independent and the split order is fixed, so results are bitwise reproducible and a row's result does not
 // depend on the other rows of the call.
 #pragma once
@@ -89,13 +89,19 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// e4m3 byte pair HI of w (0..15 each) -> the two bf16 integers
+// INT4: the 128 terms of a group, up to 15 |x| each, could leave fp32's range where |x| reaches 2^116 although the output
+// (scales are small) does not. So nibbles and sums of x carry a factor 2^-11, taken back once from the finished sums: no
+// finite x overflows, and at the other end products of the smallest normal x (2^-137) are subnormals that the matrix cores
+// keep, 2^-149 apart.
+constexpr float kI4Scale = 0.25f, kI4Back = 2048.0f;   // q 2^-9 as e4m3, times 2^-2
+constexpr uint32_t kI4Ones = 0x3A003A00u;              // a bf16 pair of 2^-11
+
+// e4m3 byte pair HI of w (0..15 each) -> the two integers times 2^-11, as bf16
 template <bool HI>
 __device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w)
 {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 512.0f, HI));
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, kI4Scale, HI));
 }
-
 // P tiles per unit, S waves sharing them along K (W / S units per block), D stages in flight per wave, MT activation
 // rows staged (4, 8 or 16 >= M), AUX cache policy of the weight loads, IL: a unit's waves take the stages in turn
 // (neighbouring waves read neighbouring bytes of a row) rather than a contiguous range each.
@@ -248,15 +254,14 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
             *reinterpret_cast<u32x4*>(lds + kXBytes + (uint32_t)(t2 % kSlots) * kSlotBytes +
                                       w_at(i * WR + lane / WP, lane % WP)) = B.w[t2][i];
     };
-    const uint32_t one2 = (uint32_t)__builtin_amdgcn_readfirstlane(0x3F803F80);
+    const uint32_t one2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)kI4Ones);
     const u32x4 ones = {one2, one2, one2, one2};
     auto mfma = [](const u32x4 a, const u32x4 b, const f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                        0, 0);
     };
-    // INT4: this lane's metadata words. Rows past N and tiles past the unit's read words that nothing wrote: their weights
-    // are zero and their outputs are not stored, but a NaN there must not reach the other tiles (it cannot: tiles and D
-    // columns are independent).
+    // INT4: this lane's metadata words. Rows past N and tiles past the unit's read words that nothing wrote; their sums are
+    // meaningless, stay in their own D columns and are not stored.
     const uint32_t* mw = md + (I4 ? (t0 - bt0) * kTileRows + ln : 0);
 
     f32x4 acc[P];
@@ -359,6 +364,7 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
             const int m = 4 * lh + c;
             if (m >= p.M) continue;
             float o = v[c];
+            if constexpr (I4) o = o * kI4Back;
             if constexpr (F == kFP8) o = o * __uint_as_float(ep_scale[e]);
             if (p.bias) o = o + bf16_to_f32(ep_bias[e]);
             p.y[(size_t)m * (size_t)p.N + (size_t)ep_row[e]] = (uint16_t)f32_to_bf16_out(o);

@@ -8,37 +8,70 @@
 namespace paia {
 namespace {
 
-constexpr int kMaxP = 6;
+// Launch shapes, each a sweep's choice over N = 3584..128256, K = 512..18944 (us on MI355X):
+//   * W waves split the K of P tiles. BF16 and FP8 run best as 4-wave blocks, several to a CU, so that one block's start and
+//     end lie under another's stream (FP8 28672x4096 M = 16 20.6 with 4 waves, 21.5 with 8; 10112x4096 10.0 / 11.1; BF16
+//     33000x2048 22.6 / 26.0); but a BF16 row beyond 8 KiB keeps one 4-wave block per CU from having enough in flight
+//     (9216x8192 M = 8 34.9 with 4 waves, 26.4 with 8; 4096x14336 M = 4 21.1 / 20.5). INT4 spends as long on decoding a stage as on reading it and wants more waves on it
+//     (4096x14336 M = 4 9.9 with 8 waves, 12.4 with 4), except for short rows, which leave 8 waves a stage or none each
+//     (100000x512 M = 4 9.4 with 4, 12.1 with 8; one tile per CU: 300x1024 2.86 / 2.95, but 2048x2048 3.72 / 3.53).
+//   * D stages in flight. One tile per wave: the stages of a K = 4096 row at once (FP8 4096x4096 M = 4 5.06 with four, 5.6
+//     with two), two for FP8 at 16 activation rows (registers) and for INT4 up to 8 stages per wave (4096x4096 4.97 /
+//     5.16 with four; 4096x14336 10.98 / 9.49). More tiles need fewer, and a second stage soon costs more registers than it
+//     brings bytes (FP8 28672x4096 M = 16 P = 4 20.6 with one, 21.5 with two).
+//   * FP8 and BF16 weights stream (nt); an INT4 row's 64 bytes share a 128-byte line with the next stage's, which the default
+//     policy keeps (4096x14336 M = 4 10.8 against 11.9).
+//   * The stages go to the waves in turn for one tile per wave and for INT4 (28672x4096 M = 4 15.8, 17.1 in contiguous
+//     ranges), in contiguous ranges otherwise (FP8 14336x4096 M = 16 12.6, 13.3 in turn).
+constexpr int kShortK = 2560, kLongBf16K = 4096;
 
-// Launch shapes: 8 waves split K of P tiles. Stages in flight, D: with one tile per wave all the stages of a K = 4096 row
-// (FP8 4096x4096 M = 4: 5.06 us with four, 5.6 with two); INT4's take half the bytes but more decode, and two are enough up
-// to 8 stages per wave (4096x4096 4.97 us with two, 5.16 with four; 4096x14336 10.98 with two, 9.49 with four; at 16
-// activation rows three, 14.9, for the registers). From P = 3 on one stage of P tiles is enough in flight and a second one
-// only costs registers (FP8 9216x8192 M = 16 16.5 us either way, 10112x4096 10.4 against 10.6). FP8 and BF16 weights stream
-// (nt); an INT4 row's 64 bytes share a 128-byte line with the next stage's, which the default policy keeps (4096x14336
-// M = 4 10.8 us against 11.9). The stages go to the waves in turn for P <= 2 and for INT4 (gate_up 28672x4096 M = 4: 15.8 us
-// in turn, 17.1 in contiguous ranges), in contiguous ranges for the wide BF16 and FP8 launches (FP8 14336x4096 M = 16 12.6
-// us against 13.3).
-template <int F, int MT, int P, int D>
+template <int F, int MT, int P, int W, int D>
 int launch_d(const BatchParams& b, int blocks, hipStream_t st)
 {
     constexpr bool I4 = TileFmt<F>::kI4F;
-    return launch_tile<F, P, 8, 8, D, MT, I4 ? 0 : 2, I4 || P <= 2>(b, blocks, st);
+    return launch_tile<F, P, W, W, D, MT, I4 ? 0 : 2, I4 || P == 1>(b, blocks, st);
 }
 template <int F, int MT, int P>
 int launch_p(const BatchParams& b, int blocks, hipStream_t st)
 {
-    if constexpr (P == 1 && TileFmt<F>::kI4F) {
-        if (b.K <= 64 * TileFmt<F>::kCols) return launch_d<F, MT, 1, 2>(b, blocks, st);
-        return launch_d<F, MT, 1, MT == 16 ? 3 : 4>(b, blocks, st);
+    if constexpr (TileFmt<F>::kI4F) {
+        if constexpr (P <= 4) {
+            if (b.K <= (P == 1 ? 1024 : kShortK)) return launch_d<F, MT, P, 4, P <= 2 ? 2 : 1>(b, blocks, st);
+        }
+        if constexpr (P == 1) {
+            if (b.K > 64 * TileFmt<F>::kCols) return launch_d<F, MT, 1, 8, MT == 16 ? 3 : 4>(b, blocks, st);
+        }
+        return launch_d<F, MT, P, 8, P <= 2 ? 2 : 1>(b, blocks, st);
     } else {
-        return launch_d<F, MT, P, P == 1 ? 4 : (P == 2 ? 2 : 1)>(b, blocks, st);
+        if constexpr (F == kBF16 && P <= 3) {
+            if (b.K > kLongBf16K && blocks == 0) return launch_d<F, MT, P, 8, P == 1 ? 4 : (P == 2 ? 2 : 1)>(b, blocks, st);
+        }
+        constexpr int D = P == 1 ? (F == kFP8 && MT == 16 ? 2 : 4) : (P <= 3 || (P == 4 && MT <= 8) ? 2 : 1);
+        return launch_d<F, MT, P, 4, D>(b, blocks, st);
     }
 }
 
 template <int F, int MT>
-int launch_mt(const BatchParams& b, int P, int blocks, hipStream_t st)
+int launch_mt(const BatchParams& b, hipStream_t st)
 {
+    const int cus = device_facts().cus > 0 ? device_facts().cus : 256;
+    const int ntiles = (b.N + kTileRows - 1) / kTileRows;
+    int P = (ntiles + cus - 1) / cus, blocks = 0;
+    if (!TileFmt<F>::kI4F && MT == 4 && ntiles > 4 * cus && b.K > kShortK) {
+        // few activation rows: x is cheap to bring in again for every tile, and a block per tile balances best (FP8
+        // 28672x4096 M = 4 18.7 against 19.4 for the best P > 1, BF16 33.9 / 34.7, FP8 128256x4096 73.0 / 74.2)
+        P = 1;
+        blocks = ntiles;
+    } else if (P > (b.K <= kShortK ? 4 : 6)) {
+        // beyond one block per CU: rounds of two blocks per CU of at most five tiles, for short rows of three of at most
+        // four; the fewest blocks where nearly all of them then take P tiles (28672x4096 INT4: 448 of 4 tiles 15.0, 512 of 3
+        // or 4 15.4; 33000x2048 needs all 768)
+        const int per_round = (b.K <= kShortK ? 3 : 2) * cus, most = b.K <= kShortK ? 4 : 5;
+        blocks = per_round * ((ntiles + per_round * most - 1) / (per_round * most));
+        P = (ntiles + blocks - 1) / blocks;
+        const int fewest = (ntiles + P - 1) / P;
+        if (8 * fewest >= 7 * blocks) blocks = fewest;
+    }
     switch (P) {
     case 1: return launch_p<F, MT, 1>(b, blocks, st);
     case 2: return launch_p<F, MT, 2>(b, blocks, st);
@@ -52,21 +85,9 @@ int launch_mt(const BatchParams& b, int P, int blocks, hipStream_t st)
 template <int F>
 int launch_fmt(const BatchParams& b, hipStream_t st)
 {
-    const int cus = device_facts().cus > 0 ? device_facts().cus : 256;
-    const int ntiles = (b.N + kTileRows - 1) / kTileRows;
-    // one block per CU while P <= 6 covers the tiles, else rounds of two blocks per CU with P <= 5; fewer blocks where all
-    // but the last take P tiles anyway (28672x4096: 448 of 4 tiles 15.0 us, 512 of 3 or 4 15.4; 33000x2048 needs the 512:
-    // 413 of 5 tiles leave 99 CUs with one block and 157 with two)
-    int P = (ntiles + cus - 1) / cus, blocks = 0;
-    if (P > kMaxP) {
-        blocks = 2 * cus * ((ntiles + 2 * cus * 5 - 1) / (2 * cus * 5));
-        P = (ntiles + blocks - 1) / blocks;
-        const int fewest = (ntiles + P - 1) / P;
-        if (8 * fewest >= 7 * blocks) blocks = fewest;
-    }
-    if (b.M <= 4) return launch_mt<F, 4>(b, P, blocks, st);
-    if (b.M <= 8) return launch_mt<F, 8>(b, P, blocks, st);
-    return launch_mt<F, 16>(b, P, blocks, st);
+    if (b.M <= 4) return launch_mt<F, 4>(b, st);
+    if (b.M <= 8) return launch_mt<F, 8>(b, st);
+    return launch_mt<F, 16>(b, st);
 }
 
 }  // namespace

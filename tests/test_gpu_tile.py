@@ -1,0 +1,109 @@
+"""GPU parity of the tile kernel (gemv_tile.h: the small-batch entry points with the variant left to the library) against
+the CPU oracle, at the edges of its launch rule: one to six tiles of 16 rows per wave and more than one round of blocks,
+rows that end inside a tile and inside a stage, one stage for many waves, long K, odd group counts, and metadata that is not
+aligned for the wide loads. Bars as for the other small-batch kernels (test_gpu_batch.py)."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import make, note
+from paia_bench.inputs import to_device
+from test_gpu_batch import check_rows, oracle_rows, run_batch, x_rows, xbits
+
+pytestmark = pytest.mark.gpu
+
+# (N, K / the format's K step, M): tiles on a 256-CU GPU 1, 2, 256, 257, 700, 1100, 1300, 1600 and 3200
+EDGES = [(1, 1, 16), (17, 3, 3), (33, 9, 5), (4096, 5, 9), (4097, 2, 16), (11200, 3, 4), (17593, 2, 8), (20800, 1, 16),
+         (25600, 3, 6), (51200, 1, 3), (48, 130, 16), (70, 67, 7), (20800, 21, 4)]
+STEP = {"bf16": 72, "fp8": 144, "int4": 128, "int4zp": 128}   # BF16 and FP8: stages of 64 and 128 columns with a tail
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "int4", "int4zp"])
+@pytest.mark.parametrize("N,kq,M", EDGES)
+def test_edges(oracle, gemv_lib, cuda, fmt, N, kq, M):
+    K = STEP[fmt] * kq
+    ops, np_ops = make(fmt, N, K, bias=fmt != "int4")
+    dev = to_device(ops, cuda)
+    x = x_rows(M, K, 6000 + M + N + K)
+    rows = np.unique(np.concatenate([np.arange(0, N, max(1, N // 150)), np.arange(max(0, N - 17), N)])).astype(np.int64)
+    refs = oracle_rows(oracle, fmt, np_ops, xbits(x), rows)
+    note(f"tile {fmt} M={M} N={N} K={K}")
+    buf = torch.full((M * N + 64,), float("nan"), dtype=torch.bfloat16, device=cuda)
+    y = run_batch(gemv_lib, fmt, dev, x.to(cuda), y=buf[:M * N].view(M, N))
+    torch.cuda.synchronize()
+    assert not torch.isnan(y).any() and torch.isnan(buf[M * N:]).all()
+    check_rows(oracle, y, refs, f"tile {fmt} M={M} {N}x{K}", rows)
+
+
+@pytest.mark.parametrize("fmt", ["int4", "int4zp"])
+@pytest.mark.parametrize("off", [0, 2, 6, 8])
+def test_metadata_alignment(gemv_lib, cuda, fmt, off):
+    """Scales and zero points at any alignment of the contract (2 bytes and 1): bit for bit the aligned call's result."""
+    N, K, M = 4112, 1024, 8
+    ops, _ = make(fmt, N, K)
+    dev = to_device(ops, cuda)
+    x = x_rows(M, K, 77).to(cuda)
+    note(f"tile metadata {fmt} offset {off}")
+    want = run_batch(gemv_lib, fmt, dev, x)
+    moved = dict(dev)
+    s = torch.zeros(dev["scales"].numel() + 8, dtype=dev["scales"].dtype, device=cuda)
+    moved["scales"] = s[off // 2: off // 2 + dev["scales"].numel()].copy_(dev["scales"].view(-1)).view(dev["scales"].shape)
+    if fmt == "int4zp":
+        z = torch.zeros(dev["zeros"].numel() + 16, dtype=torch.uint8, device=cuda)
+        o = off + (off == 6)   # an odd address too
+        moved["zeros"] = z[o: o + dev["zeros"].numel()].copy_(dev["zeros"].view(-1)).view(dev["zeros"].shape)
+    got = run_batch(gemv_lib, fmt, moved, x)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "int4", "int4zp"])
+def test_replays_and_rows(gemv_lib, cuda, fmt):
+    """Captured and replayed with eager work between the replays, and with other activation rows beside it: every result
+    bit for bit the eager one (the split order is fixed and a row does not depend on its neighbours)."""
+    N, K, M = 6150, 2048, 12
+    ops, _ = make(fmt, N, K, bias=fmt != "int4")
+    dev = to_device(ops, cuda)
+    x = x_rows(M, K, 9).to(cuda)
+    note(f"tile replays {fmt}")
+    eager = run_batch(gemv_lib, fmt, dev, x)
+    torch.cuda.synchronize()
+    x2 = torch.cat([x[:9], x_rows(7, K, 10).to(cuda) * 100]).contiguous()
+    y2 = run_batch(gemv_lib, fmt, dev, x2)
+    torch.cuda.synchronize()
+    assert torch.equal(y2[:9].view(torch.int16), eager[:9].view(torch.int16))
+    y = torch.empty_like(eager)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run_batch(gemv_lib, fmt, dev, x, y=y)
+    for i in range(3):
+        y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), eager.view(torch.int16)), f"replay {i}"
+        run_batch(gemv_lib, fmt, dev, x2)
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("fmt", ["int4", "int4zp"])
+@pytest.mark.parametrize("lo,hi", [(-125, -112), (-120, -55), (-50, 50), (60, 99), (100, 120)])
+def test_int4_extreme_x(oracle, gemv_lib, cuda, fmt, lo, hi):
+    """Activations over the whole bf16 range, rows of one call 2^5 apart, down to where the scaled products are subnormal and up to
+    where a group's sum of q x alone would leave fp32 (scales are divided so that the output does not): gated as the
+    reference gates."""
+    N, K, M = 321, 640, 5
+    ops, np_ops = make(fmt, N, K)
+    if hi > 99:   # 15 * 640 * 2^120 alone is beyond fp32; with scales below 2^-14 the outputs are not
+        ops["scales"] = (ops["scales"].float() * 2.0 ** -9).to(ops["scales"].dtype)
+        np_ops["scales"] = ops["scales"].view(torch.int16).numpy().view(np.uint16)
+    g = torch.Generator().manual_seed(lo * 1000 + hi)
+    e = torch.randint(lo, hi + 1, (K,), generator=g).double()
+    x0 = (1 + torch.rand(K, generator=g).double()) * torch.sign(torch.randn(K, generator=g).double()) * 2.0 ** e
+    x = torch.stack([x0 * 2.0 ** (5 * m * (1 if hi < 60 or hi > 99 and m < 2 else -1)) for m in range(M)]).to(torch.bfloat16)
+    note(f"tile extreme {fmt} {lo}..{hi}")
+    y = run_batch(gemv_lib, fmt, to_device(ops, cuda), x.to(cuda))
+    torch.cuda.synchronize()
+    for m, (r64, _) in enumerate(oracle_rows(oracle, fmt, np_ops, xbits(x))):
+        got = y[m].float().cpu().numpy().astype(np.float64)
+        assert np.isfinite(r64).all() and np.isfinite(got).all(), (m, np.abs(r64).max())
+        assert np.abs(got - r64).max() / np.abs(r64).max() < 2e-2, m
