@@ -2,17 +2,25 @@
 // GPU in one pass over W (fp32 [N][K], row-major). No reference C symbol: the reference quantizes with torch on the
 // GPU; these are the same values from hand-written gfx950 kernels.
 //
-//   FP8 rowwise  scale[n] = amax_n / 448 (1 if the row is all zero); q = e4m3_rn(clamp(w / scale, +-448)).
-//                One workgroup per row: amax by wave DPP max + LDS, then the row is re-read (from L2) and encoded
-//                four values per lane with the gfx950 OCP e4m3 convert (round to nearest even).
+//   FP8 rowwise  scale[n] = amax_n / 448 (1 if the row is all zero); q = e4m3_rn(clamp(w / scale, +-448)), the gfx950 OCP
+//                e4m3 convert (round to nearest even).
 //   INT4 g128    s16 = f16_rn(amax_g / 7) (1 if the group is all zero); sf = float(s16) (1 if it underflowed to 0);
 //                n = clamp(rint(w / sf), -7, 7) + 8, packed two per byte (weight 2j low nibble).
-//                One wave per group of 128: two values per lane, one packed byte per lane.
 //   INT4 g128 asymmetric (no reference counterpart; the format of the BASELINE INT4 configs, dequant (q - z) * s):
 //                lo = min(0, min w), hi = max(0, max w) over the group; s = bf16_rn((hi - lo) / 15) (1 if that is 0);
 //                z = clamp(rint(-lo / s), 0, 15); q = clamp(rint(w / s) + z, 0, 15). Zero points are packed two
-//                groups per byte along G, so one wave handles a pair of groups.
-// Divisions are IEEE (correctly rounded), rint rounds half to even, as torch.round and std::nearbyint do.
+//                groups per byte along G.
+// Quotients are correctly rounded, rint rounds half to even, as torch.round and std::nearbyint do.
+//
+// All three read 4 bytes and write 0.5 to 1 per weight: bound by HBM when W is read once, in 16-byte pieces, and the
+// division does not fill the VALU.
+//   FP8: the threads of a row keep it in registers between the maximum and the encoding (a wave for K <= 1024, up to 1024
+//   threads for K <= 32768; beyond, the row is read twice). With rows read twice, the second time from L2, 4096x14336 took
+//   88 us (512 KiB of rows per CU in flight is more than its share of L2) and 28672x4096 121; now 47 and 89 (6.6 TB/s).
+//   The loads are non-temporal: a row's bytes are used once (plain: 56 and 105 us).
+//   INT4: a group is 16 lanes of 8 weights, so its maximum takes four DPP steps, its scale one conversion per lane and its
+//   codes leave as 4 bytes a lane; a wave holds 8 groups. With a group per wave (2 weights and 1 byte a lane) 28672x4096 took
+//   141 us, asymmetric 183; now 96 both (5.5 TB/s). Plain loads: a lane's two 16-byte loads share lines (non-temporal 99).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -33,7 +41,6 @@ __device__ __forceinline__ float wave_max(float v)
     const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
-__device__ __forceinline__ float wave_min(float v) { return -wave_max(-v); }
 
 // four fp32 -> four e4m3 codes (byte i = value i), round to nearest even; |v| <= 448 on entry
 __device__ __forceinline__ uint32_t e4m3x4(float a, float b, float c, float d)
@@ -43,96 +50,209 @@ __device__ __forceinline__ uint32_t e4m3x4(float a, float b, float c, float d)
     return (uint32_t)w;
 }
 
-constexpr int kQBlock = 256;
-
-__global__ void __launch_bounds__(kQBlock) quantize_fp8_kernel(const float* __restrict__ W, uint8_t* __restrict__ q,
-                                                               float* __restrict__ scale, int N, int K)
+// Correctly rounded v / s from y = 1/s (correctly rounded), five multiply-adds and a sign instead of the division's
+// sequence with its own reciprocal: two residual corrections, the second of a quotient already within an ulp, which
+// Markstein's theorem makes the correctly rounded one. Needs |s| within 2^-60..2^60, so that neither y nor a residual that
+// matters leaves the normal range; quotients so small that a residual underflows round to zero in every format here.
+__device__ __forceinline__ float div_by(float v, float s, float y)
 {
-    __shared__ float red[kQBlock / kWave];
+    float q = v * y;
+    q = __builtin_fmaf(__builtin_fmaf(-s, q, v), y, q);
+    q = __builtin_fmaf(__builtin_fmaf(-s, q, v), y, q);
+    return __builtin_copysignf(q, v);   // -0 / s
+}
+__device__ __forceinline__ bool div_by_ok(float s) { return s >= 0x1p-60f && s <= 0x1p60f; }
+
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4v ld4(const float* p) { return *reinterpret_cast<const f32x4v*>(p); }
+__device__ __forceinline__ f32x4v ld4_nt(const float* p)
+{
+    return __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(p));
+}
+
+// ---- FP8: T threads per row, V float4 of the row per thread in registers (KEEP) or the row read again ----------------
+template <int T, int V, bool KEEP>
+__global__ void __launch_bounds__(T < 256 ? 256 : T) quantize_fp8_kernel(const float* __restrict__ W,
+                                                                        uint8_t* __restrict__ q,
+                                                                        float* __restrict__ scale, int N, int K)
+{
+    constexpr int kRows = T < 256 ? 256 / T : 1;   // rows per block
+    __shared__ float red[T / kWave];
+    const int tid = (int)threadIdx.x % T;
+    const int n = (int)blockIdx.x * kRows + (int)threadIdx.x / T;
+    if (kRows > 1 && n >= N) return;               // T = a wave: no barrier follows
+    const float* row = W + (size_t)n * K;
     const int K4 = K / 4;
-    for (int n = (int)blockIdx.x; n < N; n += (int)gridDim.x) {
-        const float4* row = reinterpret_cast<const float4*>(W + (size_t)n * K);
-        float amax = 0.0f;
-        for (int i = (int)threadIdx.x; i < K4; i += kQBlock) {
-            const float4 v = row[i];
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    f32x4v v[KEEP ? V : 1];
+    float amax = 0.0f;
+    auto take = [&](const f32x4v a) {
+        amax = fmaxf(amax, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            v[e] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+            if (tid + e * T < K4) v[e] = ld4_nt(row + 4 * (tid + e * T));
         }
-        amax = wave_max(amax);
+#pragma unroll
+        for (int e = 0; e < V; ++e) take(v[e]);
+    } else {
+        for (int i = tid; i < K4; i += T) take(ld4(row + 4 * i));
+    }
+    amax = wave_max(amax);
+    if constexpr (T > kWave) {
         if (lane_id() == 0) red[wave_id()] = amax;
         __syncthreads();
-        amax = red[0];
 #pragma unroll
-        for (int w = 1; w < kQBlock / kWave; ++w) amax = fmaxf(amax, red[w]);
-        __syncthreads();                                   // red is reused by the next row
-        const float s = amax > 0.0f ? amax / 448.0f : 1.0f;
-        if (threadIdx.x == 0) scale[n] = s;
-        uint32_t* qrow = reinterpret_cast<uint32_t*>(q + (size_t)n * K);
-        for (int i = (int)threadIdx.x; i < K4; i += kQBlock) {
-            const float4 v = row[i];
-            const float a = fminf(fmaxf(v.x / s, -448.0f), 448.0f), b = fminf(fmaxf(v.y / s, -448.0f), 448.0f);
-            const float c = fminf(fmaxf(v.z / s, -448.0f), 448.0f), d = fminf(fmaxf(v.w / s, -448.0f), 448.0f);
-            qrow[i] = e4m3x4(a, b, c, d);
-        }
+        for (int w = 0; w < T / kWave; ++w) amax = fmaxf(amax, red[w]);
+    }
+    const float s = amax > 0.0f ? amax / 448.0f : 1.0f;
+    if (tid == 0) scale[n] = s;
+    uint32_t* qrow = reinterpret_cast<uint32_t*>(q + (size_t)n * K);
+    const bool fast = div_by_ok(s);
+    const float y = 1.0f / s;
+    auto code = [&](const f32x4v a) -> uint32_t {
+        auto c = [&](float w) {
+            const float t = fast ? div_by(w, s, y) : w / s;
+            return fminf(fmaxf(t, -448.0f), 448.0f);
+        };
+        return e4m3x4(c(a.x), c(a.y), c(a.z), c(a.w));
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (tid + e * T < K4) qrow[tid + e * T] = code(v[e]);
+    } else {
+        for (int i = tid; i < K4; i += T) qrow[i] = code(ld4(row + 4 * i));
     }
 }
 
-// One wave per group of 128 (4 groups per 256-thread block, grid-stride over N*G groups).
+// ---- INT4: 16 lanes per group, kQSteps x 4 groups per wave -----------------------------------------------------------
+constexpr int kQBlock = 256;
+constexpr int kQSteps = 2;
+
+__device__ __forceinline__ float row16_max(float v)   // over the 16 lanes of a DPP row, in every lane of it
+{
+    v = fmaxf(v, dpp_f32<0xB1>(v));
+    v = fmaxf(v, dpp_f32<0x4E>(v));
+    v = fmaxf(v, dpp_f32<0x124>(v));
+    return fmaxf(v, dpp_f32<0x128>(v));
+}
+struct Group8 {
+    float w[8];
+};
+__device__ __forceinline__ Group8 group_load(const float* W, size_t gi, int l16, bool ok)
+{
+    f32x4v a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+    if (ok) {
+        const float* p = W + gi * 128 + (size_t)(l16 * 8);
+        a = ld4(p);
+        b = ld4(p + 4);
+    }
+    return {{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+}
+// The 8 codes of a lane as one word (weight j in nibble j).
+template <bool ZP>
+__device__ __forceinline__ uint32_t group_codes(const Group8& g, float s, float z)
+{
+    const bool fast = div_by_ok(s);
+    const float y = 1.0f / s;
+    uint32_t word = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float t = __builtin_rintf(fast ? div_by(g.w[j], s, y) : g.w[j] / s);
+        const int c = ZP ? (int)fminf(fmaxf(t + z, 0.0f), 15.0f) : (int)fminf(fmaxf(t, -7.0f), 7.0f) + 8;
+        word |= (uint32_t)c << (4 * j);
+    }
+    return word;
+}
+
 __global__ void __launch_bounds__(kQBlock) quantize_int4_kernel(const float* __restrict__ W,
                                                                 uint8_t* __restrict__ packed,
-                                                                uint16_t* __restrict__ scales, int N, int K)
+                                                                uint16_t* __restrict__ scales, size_t ngroups)
 {
-    const int G = K / 128;
-    const size_t ngroups = (size_t)N * (size_t)G;
-    const int lane = lane_id();
-    for (size_t gi = (size_t)blockIdx.x * (kQBlock / kWave) + (size_t)wave_id(); gi < ngroups;
-         gi += (size_t)gridDim.x * (kQBlock / kWave)) {
-        const size_t n = gi / (size_t)G, g = gi - n * (size_t)G;
-        const float2 v = reinterpret_cast<const float2*>(W + n * (size_t)K + g * 128)[lane];
-        const float amax = wave_max(fmaxf(fabsf(v.x), fabsf(v.y)));
+    const int lane = lane_id(), l16 = lane & 15;
+    const size_t g0 = ((size_t)blockIdx.x * (kQBlock / kWave) + (size_t)wave_id()) * (4 * kQSteps) + (size_t)(lane >> 4);
+    Group8 g[kQSteps];
+#pragma unroll
+    for (int e = 0; e < kQSteps; ++e) g[e] = group_load(W, g0 + 4 * e, l16, g0 + 4 * e < ngroups);
+#pragma unroll
+    for (int e = 0; e < kQSteps; ++e) {
+        const size_t gi = g0 + 4 * e;
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(g[e].w[j]));
+        amax = row16_max(amax);
         const _Float16 s16 = (_Float16)(amax > 0.0f ? amax / 7.0f : 1.0f);   // v_cvt_f16_f32: round to nearest even
         float sf = (float)s16;
         if (!(sf > 0.0f)) sf = 1.0f;
-        const int q0 = (int)fminf(fmaxf(__builtin_rintf(v.x / sf), -7.0f), 7.0f) + 8;
-        const int q1 = (int)fminf(fmaxf(__builtin_rintf(v.y / sf), -7.0f), 7.0f) + 8;
-        packed[n * (size_t)(K / 2) + g * 64 + (size_t)lane] = (uint8_t)(q0 | (q1 << 4));
-        if (lane == 0) scales[gi] = __builtin_bit_cast(uint16_t, s16);
+        const uint32_t word = group_codes<false>(g[e], sf, 0.0f);
+        if (gi < ngroups) {
+            reinterpret_cast<uint32_t*>(packed)[gi * 16 + (size_t)l16] = word;
+            if (l16 == 0) scales[gi] = __builtin_bit_cast(uint16_t, s16);
+        }
     }
 }
 
-// One wave per pair of groups (2j, 2j+1) of a row, so the packed zero-point byte has one writer.
+// A pair of groups (2j, 2j+1 of a row) is 32 lanes, so the packed zero-point byte has one writer: the second group's first
+// lane, or the first's where G is odd (ODD) and the pair is the row's last.
+template <bool ODD>
 __global__ void __launch_bounds__(kQBlock) quantize_int4_zp_kernel(const float* __restrict__ W,
                                                                    uint8_t* __restrict__ packed,
                                                                    uint16_t* __restrict__ scales,
-                                                                   uint8_t* __restrict__ zeros, int N, int K)
+                                                                   uint8_t* __restrict__ zeros, uint32_t npairs, int G)
 {
-    const int G = K / 128, ZB = (G + 1) / 2;
-    const size_t npairs = (size_t)N * (size_t)ZB;
-    const int lane = lane_id();
-    for (size_t pi = (size_t)blockIdx.x * (kQBlock / kWave) + (size_t)wave_id(); pi < npairs;
-         pi += (size_t)gridDim.x * (kQBlock / kWave)) {
-        const size_t n = pi / (size_t)ZB, j = pi - n * (size_t)ZB;
-        uint32_t zbyte = 0;
-        for (int h = 0; h < 2; ++h) {
-            const size_t g = 2 * j + (size_t)h;
-            if (g >= (size_t)G) break;                     // odd G: the last byte has one group (high nibble 0)
-            const float2 v = reinterpret_cast<const float2*>(W + n * (size_t)K + g * 128)[lane];
-            const float lo = fminf(wave_min(fminf(v.x, v.y)), 0.0f);
-            const float hi = fmaxf(wave_max(fmaxf(v.x, v.y)), 0.0f);
-            const float r = (hi - lo) / 15.0f;
-            uint32_t sb = f32_to_bf16_rne(r);
-            float s = bf16_to_f32(sb);
-            if (!(s > 0.0f)) {
-                sb = 0x3F80u;                              // bf16 1.0
-                s = 1.0f;
-            }
-            const float zf = fminf(fmaxf(__builtin_rintf(-lo / s), 0.0f), 15.0f);
-            const int q0 = (int)fminf(fmaxf(__builtin_rintf(v.x / s) + zf, 0.0f), 15.0f);
-            const int q1 = (int)fminf(fmaxf(__builtin_rintf(v.y / s) + zf, 0.0f), 15.0f);
-            packed[n * (size_t)(K / 2) + g * 64 + (size_t)lane] = (uint8_t)(q0 | (q1 << 4));
-            if (lane == 0) scales[n * (size_t)G + g] = (uint16_t)sb;
-            zbyte |= (uint32_t)zf << (4 * h);
+    const int lane = lane_id(), l16 = lane & 15, h = (lane >> 4) & 1;
+    const uint32_t p0 = (blockIdx.x * (kQBlock / kWave) + (uint32_t)wave_id()) * (2 * kQSteps) + (uint32_t)(lane >> 5);
+    const uint32_t ZB = (uint32_t)(G + 1) / 2;
+    Group8 g[kQSteps];
+    size_t gis[kQSteps];
+    bool ok[kQSteps], alone[kQSteps];
+#pragma unroll
+    for (int e = 0; e < kQSteps; ++e) {
+        const uint32_t pi = p0 + 2 * e;
+        alone[e] = false;
+        ok[e] = pi < npairs;
+        if constexpr (ODD) {
+            const uint32_t n = pi / ZB, j = pi - n * ZB;
+            alone[e] = 2 * j + 1 >= (uint32_t)G;
+            ok[e] = ok[e] && !(alone[e] && h);
+            gis[e] = (size_t)n * (size_t)G + 2 * j + (uint32_t)h;
+        } else {
+            gis[e] = 2 * (size_t)pi + (size_t)h;
         }
-        if (lane == 0) zeros[pi] = (uint8_t)zbyte;
+        g[e] = group_load(W, gis[e], l16, ok[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < kQSteps; ++e) {
+        float lo = g[e].w[0], hi = g[e].w[0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) {
+            lo = fminf(lo, g[e].w[j]);
+            hi = fmaxf(hi, g[e].w[j]);
+        }
+        lo = fminf(-row16_max(-lo), 0.0f);
+        hi = fmaxf(row16_max(hi), 0.0f);
+        const float r = (hi - lo) / 15.0f;
+        uint32_t sb = f32_to_bf16_rne(r);
+        float s = bf16_to_f32(sb);
+        if (!(s > 0.0f)) {
+            sb = 0x3F80u;                              // bf16 1.0
+            s = 1.0f;
+        }
+        const float zf = fminf(fmaxf(__builtin_rintf(-lo / s), 0.0f), 15.0f);
+        const uint32_t word = group_codes<true>(g[e], s, zf);
+        // the first group's zero point to the second's lanes (row_bcast:15 into rows 1 and 3)
+        const uint32_t z = (uint32_t)zf;
+        const uint32_t zfirst = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)z, 0x142, 0xA, 0xF, false);
+        if (ok[e]) {
+            reinterpret_cast<uint32_t*>(packed)[gis[e] * 16 + (size_t)l16] = word;
+            if (l16 == 0) {
+                scales[gis[e]] = (uint16_t)sb;
+                if (h) zeros[p0 + 2 * e] = (uint8_t)(zfirst | (z << 4));
+                else if (alone[e]) zeros[p0 + 2 * e] = (uint8_t)z;
+            }
+        }
     }
 }
 
@@ -141,10 +261,30 @@ __global__ void __launch_bounds__(kQBlock) quantize_int4_zp_kernel(const float* 
 namespace {
 using namespace paia;
 
-unsigned qgrid(size_t units, size_t per_block)
+// A launch has less than 2^32 threads: rows beyond kMaxBlocks blocks of 256 go into a further launch (no call on weights
+// below 4 GB needs a second).
+constexpr size_t kMaxBlocks = (size_t)1 << 23;
+
+unsigned blocks_for(size_t units, size_t per_block) { return (unsigned)((units + per_block - 1) / per_block); }
+size_t slice_rows(size_t units_per_row, size_t units_per_block)
 {
-    const size_t want = (units + per_block - 1) / per_block;
-    return (unsigned)(want < 16384 ? (want > 0 ? want : 1) : 16384);
+    const size_t r = kMaxBlocks * units_per_block / units_per_row;
+    return r > 0 ? r : 1;
+}
+
+template <int T, int V, bool KEEP>
+int launch_fp8(const void* W, void* q, void* scale, int N, int K, hipStream_t st)
+{
+    constexpr int kRows = T < 256 ? 256 / T : 1;
+    const size_t step = slice_rows(T < 256 ? 1 : T / 256, kRows);
+    for (size_t n = 0; n < (size_t)N; n += step) {
+        const size_t rows = (size_t)N - n < step ? (size_t)N - n : step;
+        hipLaunchKernelGGL((quantize_fp8_kernel<T, V, KEEP>), dim3(blocks_for(rows, kRows)), dim3(T < 256 ? 256 : T), 0, st,
+                           static_cast<const float*>(W) + n * (size_t)K, static_cast<uint8_t*>(q) + n * (size_t)K,
+                           static_cast<float*>(scale) + n, (int)rows, K);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return 0;
 }
 
 }  // namespace
@@ -154,19 +294,34 @@ extern "C" {
 int paia_quantize_fp8_rowwise(const void* W, void* q, void* scale, int N, int K, void* stream)
 {
     if (N <= 0 || K <= 0 || (K & 15) || !aligned(W, 16) || !aligned(q, 16) || !aligned(scale, 4)) return -2;
-    hipLaunchKernelGGL(quantize_fp8_kernel, dim3(qgrid((size_t)N, 1)), dim3(kQBlock), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float*>(W), static_cast<uint8_t*>(q),
-                       static_cast<float*>(scale), N, K);
-    return (int)hipGetLastError();
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    // The fewest threads that hold the row with up to 8 float4 (32 registers) each, so that rows in flight fill the chip
+    // between a row's two halves; a block for 1024 < K <= 2048, where a wave with 8 left few-row calls longer in flight
+    // (513x1040 3.5 us against 3.1).
+    if (K <= 64 * 4 * 4) return launch_fp8<64, 4, true>(W, q, scale, N, K, st);
+    if (K <= 256 * 4 * 2) return launch_fp8<256, 2, true>(W, q, scale, N, K, st);
+    if (K <= 256 * 4 * 4) return launch_fp8<256, 4, true>(W, q, scale, N, K, st);
+    if (K <= 256 * 4 * 8) return launch_fp8<256, 8, true>(W, q, scale, N, K, st);
+    if (K <= 512 * 4 * 8) return launch_fp8<512, 8, true>(W, q, scale, N, K, st);
+    if (K <= 1024 * 4 * 8) return launch_fp8<1024, 8, true>(W, q, scale, N, K, st);
+    return launch_fp8<1024, 1, false>(W, q, scale, N, K, st);
 }
 
 int paia_quantize_int4_g128(const void* W, void* packed, void* scales, int N, int K, void* stream)
 {
     if (N <= 0 || K <= 0 || (K & 127) || !aligned(W, 16) || !aligned(packed, 16) || !aligned(scales, 2)) return -2;
-    hipLaunchKernelGGL(quantize_int4_kernel, dim3(qgrid((size_t)N * (size_t)(K / 128), kQBlock / kWave)),
-                       dim3(kQBlock), 0, static_cast<hipStream_t>(stream), static_cast<const float*>(W),
-                       static_cast<uint8_t*>(packed), static_cast<uint16_t*>(scales), N, K);
-    return (int)hipGetLastError();
+    const size_t G = (size_t)K / 128;
+    constexpr size_t kPerBlock = kQBlock / kWave * 4 * kQSteps;
+    const size_t step = slice_rows(G, kPerBlock);
+    for (size_t n = 0; n < (size_t)N; n += step) {
+        const size_t ngroups = ((size_t)N - n < step ? (size_t)N - n : step) * G;
+        hipLaunchKernelGGL(quantize_int4_kernel, dim3(blocks_for(ngroups, kPerBlock)), dim3(kQBlock), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const float*>(W) + n * (size_t)K,
+                           static_cast<uint8_t*>(packed) + n * (size_t)(K / 2), static_cast<uint16_t*>(scales) + n * G,
+                           ngroups);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return 0;
 }
 
 int paia_quantize_int4_zp_g128(const void* W, void* packed, void* scales, void* zeros, int N, int K, void* stream)
@@ -174,11 +329,22 @@ int paia_quantize_int4_zp_g128(const void* W, void* packed, void* scales, void* 
     if (N <= 0 || K <= 0 || (K & 127) || !aligned(W, 16) || !aligned(packed, 16) || !aligned(scales, 2) ||
         zeros == nullptr)
         return -2;
-    const size_t pairs = (size_t)N * (size_t)((K / 128 + 1) / 2);
-    hipLaunchKernelGGL(quantize_int4_zp_kernel, dim3(qgrid(pairs, kQBlock / kWave)), dim3(kQBlock), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float*>(W), static_cast<uint8_t*>(packed),
-                       static_cast<uint16_t*>(scales), static_cast<uint8_t*>(zeros), N, K);
-    return (int)hipGetLastError();
+    const size_t G = (size_t)K / 128, ZB = (G + 1) / 2;
+    constexpr size_t kPerBlock = kQBlock / kWave * 2 * kQSteps;
+    const size_t step = slice_rows(ZB, kPerBlock);
+    for (size_t n = 0; n < (size_t)N; n += step) {
+        const size_t pairs = ((size_t)N - n < step ? (size_t)N - n : step) * ZB;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks_for(pairs, kPerBlock)), dim3(kQBlock), 0, static_cast<hipStream_t>(stream),
+                               static_cast<const float*>(W) + n * (size_t)K,
+                               static_cast<uint8_t*>(packed) + n * (size_t)(K / 2), static_cast<uint16_t*>(scales) + n * G,
+                               static_cast<uint8_t*>(zeros) + n * ZB, (uint32_t)pairs, (int)G);
+        };
+        if (G & 1) launch(quantize_int4_zp_kernel<true>);
+        else launch(quantize_int4_zp_kernel<false>);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return 0;
 }
 
 }  // extern "C"

@@ -111,6 +111,47 @@ def test_quantize_int4_zp_bitexact(oracle, gemv_lib, cuda):
         assert np.array_equal(s.cpu().view(torch.int16).numpy().view(np.uint16), s0)
 
 
+@pytest.mark.parametrize("K", [1024, 1040, 2048, 2064, 4096, 4112, 8192, 8208, 16384, 16400, 32768, 32784])
+def test_quantize_fp8_row_lengths_and_scales_bitexact(oracle, gemv_lib, cuda, K):
+    """Each row length at which the kernel changes shape, ragged in rows; scales on both sides of the exact-quotient range."""
+    rng = np.random.default_rng(K)
+    W = rng.standard_normal((7, K)) * np.array([1, 2.0 ** -54, 2.0 ** -100, 2.0 ** 68, 2.0 ** 120, 1e-38, 0.02])[:, None]
+    W = W.astype(np.float32)
+    W[:, 5] = -0.0
+    W[:, -1] *= 1.5                                        # the last column takes part in the maximum
+    note(f"quantize fp8 lengths {W.shape}")
+    q, s = run_fp8(gemv_lib, W, cuda)
+    q0, s0 = oracle.quantize_fp8_rowwise(W)
+    assert np.array_equal(s.view(np.uint32), s0.view(np.uint32)) and np.array_equal(q, q0)
+
+
+@pytest.mark.parametrize("N,K", [(1, 128), (1, 3968), (3, 4096), (11, 896), (129, 256)])
+def test_quantize_int4_ragged_groups_and_scales_bitexact(oracle, gemv_lib, cuda, N, K):
+    """Group counts that leave a wave part full (odd G too), scales past the formats' ranges, both INT4 formats."""
+    rng = np.random.default_rng(N * K)
+    G = K // 128
+    W = rng.standard_normal((N, G, 128)) * rng.choice([1e-30, 1e-9, 1e-3, 1.0, 1e4], (N, G, 1))
+    W = W.astype(np.float32).reshape(N, K)
+    W[-1, -1] = -0.0
+    d = _dev(W, cuda)
+    p = torch.empty(N, K // 2, dtype=torch.uint8, device=cuda)
+    s = torch.empty(N, G, dtype=torch.float16, device=cuda)
+    z = torch.empty(N, (G + 1) // 2, dtype=torch.uint8, device=cuda)
+    note(f"quantize int4 ragged {N}x{K}")
+    gemv_lib.quantize_int4_g128(d.data_ptr(), p.data_ptr(), s.data_ptr(), N, K)
+    torch.cuda.synchronize()
+    p0, s0 = oracle.quantize_int4_g128(W)
+    assert np.array_equal(s.cpu().view(torch.int16).numpy().view(np.uint16), s0) and np.array_equal(p.cpu().numpy(), p0)
+    W *= np.where(np.arange(K) // 128 % 2, np.float32(1e18), np.float32(1))   # bf16 scales keep fp32's range
+    d = _dev(W, cuda)
+    s = s.view(torch.bfloat16)
+    gemv_lib.quantize_int4_zp_g128(d.data_ptr(), p.data_ptr(), s.data_ptr(), z.data_ptr(), N, K)
+    torch.cuda.synchronize()
+    p0, s0, z0 = oracle.quantize_int4_zp_g128(W)
+    assert np.array_equal(p.cpu().numpy(), p0) and np.array_equal(z.cpu().numpy(), z0)
+    assert np.array_equal(s.cpu().view(torch.int16).numpy().view(np.uint16), s0)
+
+
 def test_quant_api_on_device_matches_definition(cuda):
     """paia_gemv.quant on a GPU tensor (the HIP kernels through the torch ops) == the torch definition on the CPU."""
     from paia_gemv import quant
