@@ -58,6 +58,24 @@ def test_dequant_bitexact_seeded(oracle, gemv_lib, cuda, fmt):
         assert_same_floats(out.cpu().numpy(), want, f"{fmt} {N}x{K}")
 
 
+@pytest.mark.parametrize("fmt,N,K", [("fp8", 515, 16), ("fp8", 9, 1360), ("fp8", 3, 2048), ("fp8", 2, 2064),
+                                     ("fp8", 5, 4112), ("int4", 65, 128), ("int4", 4, 2048), ("int4", 3, 4224),
+                                     ("int4zp", 33, 896), ("int4zp", 7, 1920), ("int4zp", 2, 8320)])
+def test_dequant_block_edges_bitexact(oracle, gemv_lib, cuda, fmt, N, K):
+    """Rows per block (K <= 2048, the last block part full) and blocks per row (the last part full); nothing past the end."""
+    ops, np_ops = make(fmt, N, K)
+    dev = to_device(ops, cuda)
+    out = torch.full((N * K + 4096,), -7.0, dtype=torch.float32, device=cuda)
+    note(f"dequant {fmt} edges {N}x{K}")
+    names = {"fp8": ("Wq", "scale"), "int4": ("Wq", "scales"), "int4zp": ("Wq", "scales", "zeros")}[fmt]
+    fn = {"fp8": "dequant_fp8", "int4": "dequant_int4", "int4zp": "dequant_int4_zp"}[fmt]
+    getattr(gemv_lib, fn)(*(dev[n].data_ptr() for n in names), out.data_ptr(), N, K)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert_same_floats(got[:N * K].reshape(N, K), getattr(oracle, fn)(*(np_ops[n] for n in names)), f"{fmt} {N}x{K}")
+    assert np.all(got[N * K:] == -7.0)
+
+
 def test_dequant_int4zp_odd_group_count(oracle, gemv_lib, cuda):
     """G odd (K = 384, 640): the last zero byte holds one group in its low nibble."""
     for N, K in [(5, 384), (17, 640)]:
