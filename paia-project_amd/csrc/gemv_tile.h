@@ -72,11 +72,12 @@ struct TileFmt {
 // A wave's private LDS: one stage of x (MT rows), then the stage's weights of two tiles (in order within the wave: the
 // third tile's weights overwrite the first's behind their reads), reused for the wave's P partial tiles at the end.
 constexpr int kTileSlots = 2;
-template <int F, int P, int MT>
+// RING: the last two 128-byte lines of each of the P tiles' rows instead.
+template <int F, int P, int MT, bool RING>
 __host__ __device__ constexpr uint32_t tile_wave_bytes()
 {
     const uint32_t x = (uint32_t)MT * 2u * TileFmt<F>::kCols;
-    const uint32_t w = (uint32_t)(P < kTileSlots ? P : kTileSlots) * kTileRows * TileFmt<F>::kRowBytes;
+    const uint32_t w = (uint32_t)(RING ? 2 * P : (P < kTileSlots ? P : kTileSlots)) * kTileRows * TileFmt<F>::kRowBytes;
     return x + w > (uint32_t)P * 1024u ? x + w : (uint32_t)P * 1024u;
 }
 
@@ -102,10 +103,14 @@ __device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w)
 {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, kI4Scale, HI));
 }
+
 // P tiles per unit, S waves sharing them along K (W / S units per block), D stages in flight per wave, MT activation
 // rows staged (4, 8 or 16 >= M), AUX cache policy of the weight loads, IL: a unit's waves take the stages in turn
 // (neighbouring waves read neighbouring bytes of a row) rather than a contiguous range each.
-template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL>
+// RING (BF16, FP8; not IL): for rows that are no multiple of 128 bytes, where a stage's 128 bytes of a row lie in two lines
+// and each line would be read twice (and fetched 1.6 times: with nt it is gone by the second read). A wave reads the lines of
+// its range once each, whole, and a stage takes its columns from the row's last two lines in LDS.
+template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL, bool RING>
 __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams p)
 {
     using T = TileFmt<F>;
@@ -115,11 +120,12 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     constexpr int WP = RB / 16, WR = kWave / WP;      // 16-byte pieces per weight row and stage, rows per load
     constexpr int XP = 2 * C / 16;                    // 16-byte pieces per x row and stage
     constexpr int kUnits = W / S;
-    constexpr int kSlots = P < kTileSlots ? P : kTileSlots;
-    constexpr uint32_t kXBytes = (uint32_t)MT * 2u * C, kSlotBytes = (uint32_t)kTileRows * RB;
-    constexpr uint32_t kWaveBytes = tile_wave_bytes<F, P, MT>();
+    constexpr int kSlots = RING || P < kTileSlots ? P : kTileSlots;
+    constexpr uint32_t kXBytes = (uint32_t)MT * 2u * C, kSlotBytes = (uint32_t)kTileRows * RB * (RING ? 2u : 1u);
+    constexpr uint32_t kWaveBytes = tile_wave_bytes<F, P, MT, RING>();
     constexpr int kOuts = (kUnits * P + W - 1) / W;   // tiles a wave reduces and stores
     static_assert(W % S == 0 && (MT == 4 || MT == 8 || MT == 16), "launch shape");
+    static_assert(!RING || (!I4 && !IL), "lines of contiguous ranges");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
     const int lane = lane_id(), wave = wave_id();
@@ -137,7 +143,9 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     const int t0 = tile_at(u0 + unit), nt = tile_at(u0 + unit + 1) - t0;   // this unit's tiles, nt <= P
     const int k0 = IL ? split : split * p.stages / S;
     const int n = IL ? (p.stages - split + S - 1) / S : (split + 1) * p.stages / S - k0;   // this wave's stages
-    auto stage_at = [&](int t) { return IL ? k0 + t * S : k0 + t; };
+    // RING: line t = 0 only fills the ring, line t > 0 completes stage t - 1 of the range
+    const int nl = RING ? (n > 0 ? n + 1 : 0) : n;
+    auto stage_at = [&](int t) { return IL ? k0 + t * S : (RING ? k0 + t - 1 : k0 + t); };
 
     // INT4 metadata of the block's rows: item i is four groups of one row
     const int bt0 = tile_at(u0), brows = I4 ? max(0, min((tile_at(u0 + kUnits) - bt0) * kTileRows, p.N - bt0 * kTileRows)) : 0;
@@ -206,7 +214,10 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
         rw[t] = make_rsrc(p.W + (rows ? (size_t)row0 : 0) * p.row_bytes, rows * p.row_bytes);
     }
     const __amdgpu_buffer_rsrc_t xrs = make_rsrc(p.x, (uint32_t)p.M * (uint32_t)p.K * 2u);
-    const uint32_t lw = (uint32_t)(lane / WP) * p.row_bytes + (uint32_t)(lane % WP) * 16u;
+    // RING: the row's first byte in its first line (lines counted from the tile's first byte, so that none starts before it;
+    // 8 rows are a multiple of 128 bytes, so a row's is that of its lane group)
+    const uint32_t ws = RING ? ((uint32_t)(lane / WP) * p.row_bytes) & 127u : 0u;
+    const uint32_t lw = (uint32_t)(lane / WP) * p.row_bytes - ws + (uint32_t)(lane % WP) * 16u;
     const uint32_t lx = (uint32_t)(lane / XP) * (uint32_t)p.K * 2u + (uint32_t)(lane % XP) * 16u;
     const int cw = (lane % WP) * (C / WP), cx = (lane % XP) * 8;     // first column of the lane's 16 bytes
     const uint32_t wstep = (uint32_t)WR * p.row_bytes, xstep = (uint32_t)XR * (uint32_t)p.K * 2u;
@@ -218,9 +229,15 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     // Unconditional loads (a load under a branch makes the compiler wait for every outstanding one); t >= n: none in range.
     auto issue = [&](Stage& B, int t) {
         const int kb = stage_at(t);
-        const int left = t < n ? p.K - kb * C : 0;     // columns from the stage's first one on
-        const uint32_t wo = cw < left ? lw + (uint32_t)kb * (uint32_t)RB : kOOB;
-        const uint32_t xo = cx < left ? lx + (uint32_t)kb * (uint32_t)(2 * C) : kOOB;
+        const int left = t < nl ? p.K - kb * C : 0;    // columns from the stage's first one on
+        uint32_t wo;
+        if constexpr (RING) {   // line kb + 1 of the rows; bytes past a row's end read zero
+            const int wl = t < nl ? (int)p.row_bytes - (kb + 1) * RB : -RB;
+            wo = (lane % WP) * 16 - (int)ws < wl ? lw + (uint32_t)(kb + 1) * (uint32_t)RB : kOOB;
+        } else {
+            wo = cw < left ? lw + (uint32_t)kb * (uint32_t)RB : kOOB;
+        }
+        const uint32_t xo = cx < left && (!RING || t > 0) ? lx + (uint32_t)kb * (uint32_t)(2 * C) : kOOB;
 #pragma unroll
         for (int j = 0; j < XL; ++j) B.x[j] = ld16<0>(xrs, xo + xstep * (uint32_t)j, 0u);
 #pragma unroll
@@ -248,11 +265,22 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
                          : (uint32_t)(row * 64 + ((piece ^ ((row >> 1) & 3)) << 4));
     };
     auto x_at = [](int row, int piece) -> uint32_t { return (uint32_t)(row * 2 * C + ((piece ^ (row & 7)) << 4)); };
-    auto put_w = [&](const Stage& B, int t2) {
+    // RING: 16 pieces a row, a line's in one half, turned back by the line's part before the row and on by the row: a stage's
+    // piece then lies at a place that does not depend on the alignment, the 16 rows' in 16 different bank groups
+    const uint32_t ring_put = (uint32_t)(lane % WP) + (uint32_t)(lane / WP) - (ws >> 4);
+    auto put_w = [&](const Stage& B, int t2, int t) {
 #pragma unroll
-        for (int i = 0; i < L; ++i)
-            *reinterpret_cast<u32x4*>(lds + kXBytes + (uint32_t)(t2 % kSlots) * kSlotBytes +
-                                      w_at(i * WR + lane / WP, lane % WP)) = B.w[t2][i];
+        for (int i = 0; i < L; ++i) {
+            const uint32_t at = RING ? (uint32_t)(i * WR + lane / WP) * 256u +
+                                           (((ring_put + (uint32_t)(i * WR) + 8u * (uint32_t)(t & 1)) & 15u) << 4)
+                                     : w_at(i * WR + lane / WP, lane % WP);
+            *reinterpret_cast<u32x4*>(lds + kXBytes + (uint32_t)(t2 % kSlots) * kSlotBytes + at) = B.w[t2][i];
+        }
+    };
+    auto get_w = [&](int t2, int i, int t) {
+        const uint32_t at = RING ? (uint32_t)ln * 256u + (((uint32_t)(4 * i + lh + ln) + 8u * (uint32_t)((t + 1) & 1)) & 15u) * 16u
+                                 : w_at(ln, 4 * i + lh);
+        return *reinterpret_cast<const u32x4*>(lds + kXBytes + (uint32_t)(t2 % kSlots) * kSlotBytes + at);
     };
     const uint32_t one2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)kI4Ones);
     const u32x4 ones = {one2, one2, one2, one2};
@@ -276,7 +304,7 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
             if (XR <= MT || lane < MT * XP) *reinterpret_cast<u32x4*>(lds + x_at(j * XR + lane / XP, lane % XP)) = v;
         }
 #pragma unroll
-        for (int t2 = 0; t2 < kSlots; ++t2) put_w(B, t2);
+        for (int t2 = 0; t2 < kSlots; ++t2) put_w(B, t2, t);
         wave_lds_order();
         u32x4 a[X];
 #pragma unroll
@@ -296,12 +324,10 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
             u32x4 w[L];
             if (t2 >= kSlots) wave_lds_order();
 #pragma unroll
-            for (int i = 0; i < L; ++i)
-                w[i] = *reinterpret_cast<const u32x4*>(lds + kXBytes + (uint32_t)(t2 % kSlots) * kSlotBytes +
-                                                       w_at(ln, 4 * i + lh));
+            for (int i = 0; i < L; ++i) w[i] = get_w(t2, i, t);
             if (t2 + kSlots < P) {
                 wave_lds_order();
-                put_w(B, t2 + kSlots);
+                put_w(B, t2 + kSlots, t);
             }
             if constexpr (F == kBF16) {
 #pragma unroll
@@ -334,18 +360,26 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
 
     // D stages are in flight throughout; a stage's buffer is refilled as soon as it is consumed. The last D stages are
     // consumed without a refill (a round of empty loads would queue behind the CU's outstanding ones).
-    int t = 0;
-    for (; t + D < n; t += D) {
+    constexpr int kFirst = RING ? 1 : 0;   // the first line's buffer moves on at once
+    if constexpr (RING) {
+#pragma unroll
+        for (int t2 = 0; t2 < P; ++t2) put_w(buf[0], t2, 0);
+        wave_lds_order();
+        issue(buf[0], D);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int t = kFirst;
+    for (; t + D < nl; t += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            consume(buf[d], t + d);   // t + d < n: the loop's condition
-            issue(buf[d], t + d + D);
+            consume(buf[(d + kFirst) % D], t + d);   // t + d < nl: the loop's condition
+            issue(buf[(d + kFirst) % D], t + d + D);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (t + d < n) consume(buf[d], t + d);
+        if (t + d < nl) consume(buf[(d + kFirst) % D], t + d);
 
     // Partial tiles to the wave's own region, one barrier, then (unit, tile) q is added up in split order and stored.
 #pragma unroll
@@ -381,7 +415,7 @@ constexpr int kTileRefused = -100;
 
 // The launch on `st` with `blocks` blocks (raised to one per kUnits * P tiles). Returns 0, kTileRefused when the block's
 // metadata does not fit the LDS, or a hipError_t.
-template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL>
+template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL, bool RING>
 int launch_tile(const BatchParams& b, int blocks, hipStream_t st)
 {
     constexpr int kUnits = W / S;
@@ -416,9 +450,9 @@ int launch_tile(const BatchParams& b, int blocks, hipStream_t st)
         if (lds > rows_max_lds()) return kTileRefused;
     }
     p.wave_off = (uint32_t)lds;
-    lds += (uint64_t)W * tile_wave_bytes<F, P, MT>();
+    lds += (uint64_t)W * tile_wave_bytes<F, P, MT, RING>();
     if (lds > rows_max_lds()) return kTileRefused;
-    auto kernel = &gemv_tile_kernel<F, P, W, S, D, MT, AUX, IL>;
+    auto kernel = &gemv_tile_kernel<F, P, W, S, D, MT, AUX, IL, RING>;
     if (lds > kMaxLds) {   // beyond the default dynamic-LDS limit: raise it once per device for this kernel
         static std::atomic<uint64_t> raised{0};
         int dev = 0;

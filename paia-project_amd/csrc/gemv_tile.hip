@@ -25,11 +25,32 @@ namespace {
 //     ranges), in contiguous ranges otherwise (FP8 14336x4096 M = 16 12.6, 13.3 in turn).
 constexpr int kShortK = 2560, kLongBf16K = 4096;
 
+// Rows that are no multiple of 128 bytes (BF16, FP8): every stage's bytes of a row lie in two lines. Read line by line where
+// a wave's range pays for its extra line (RING); else plain loads in turn, so that the second stage of a line finds it in
+// cache (nt fetched 1.6 times the weights' bytes: BF16 45653x10952 M = 11 250 us, plain in turn 204, RING 155; FP8
+// 72800x7024 M = 16 152 / 119 / 100). Several tiles per wave: down to 1280-byte rows (BF16 21595x664 M = 16 9.5 RING, 10.3
+// plain; 30000x520 12.2 / 10.7). One tile, which waits on latency more than it streams: K >= 4096 and more than 32 tiles
+// (FP8 4000x4944 M = 16 8.6 / 8.8, 1000x3600 6.5 / 4.8; BF16 600x18936 M = 8 22.9 / 28.0, 50x15016 M = 11 20.6 / 14.9).
+enum { kLines, kRing, kSplit };
+template <int P>
+int row_form(const BatchParams& b)
+{
+    if (b.row_bytes % 128 == 0) return kLines;
+    return (P == 1 ? b.K >= 4096 && b.N > 32 * kTileRows : b.row_bytes >= 1280) ? kRing : kSplit;
+}
+
 template <int F, int MT, int P, int W, int D>
 int launch_d(const BatchParams& b, int blocks, hipStream_t st)
 {
-    constexpr bool I4 = TileFmt<F>::kI4F;
-    return launch_tile<F, P, W, W, D, MT, I4 ? 0 : 2, I4 || P == 1>(b, blocks, st);
+    if constexpr (TileFmt<F>::kI4F) {
+        return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);
+    } else {
+        switch (row_form<P>(b)) {
+        case kLines: return launch_tile<F, P, W, W, D, MT, 2, P == 1, false>(b, blocks, st);
+        case kRing: return launch_tile<F, P, W, W, D, MT, 2, false, true>(b, blocks, st);
+        default: return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);
+        }
+    }
 }
 template <int F, int MT, int P>
 int launch_p(const BatchParams& b, int blocks, hipStream_t st)
@@ -57,9 +78,12 @@ int launch_mt(const BatchParams& b, hipStream_t st)
     const int cus = device_facts().cus > 0 ? device_facts().cus : 256;
     const int ntiles = (b.N + kTileRows - 1) / kTileRows;
     int P = (ntiles + cus - 1) / cus, blocks = 0;
-    if (!TileFmt<F>::kI4F && MT == 4 && ntiles > 4 * cus && b.K > kShortK) {
+    if (!TileFmt<F>::kI4F && MT == 4 && ntiles > 4 * cus && b.K > kShortK &&
+        (b.row_bytes % 128 == 0 || ntiles <= 16 * cus)) {
         // few activation rows: x is cheap to bring in again for every tile, and a block per tile balances best (FP8
-        // 28672x4096 M = 4 18.7 against 19.4 for the best P > 1, BF16 33.9 / 34.7, FP8 128256x4096 73.0 / 74.2)
+        // 28672x4096 M = 4 18.7 against 19.4 for the best P > 1, BF16 33.9 / 34.7, FP8 128256x4096 73.0 / 74.2); rows with
+        // split lines up to 4096 tiles, where their one extra line per range is still cheaper than a longer last wave (FP8
+        // 20000x5008 M = 4 18.9 / 19.6, 40000x3008 22.6 / 24.1, but 87988x3680 61.9 / 57.1)
         P = 1;
         blocks = ntiles;
     } else if (P > (b.K <= kShortK ? 4 : 6)) {

@@ -107,3 +107,43 @@ def test_int4_extreme_x(oracle, gemv_lib, cuda, fmt, lo, hi):
         got = y[m].float().cpu().numpy().astype(np.float64)
         assert np.isfinite(r64).all() and np.isfinite(got).all(), (m, np.abs(r64).max())
         assert np.abs(got - r64).max() / np.abs(r64).max() < 2e-2, m
+
+
+# BF16 and FP8 row lengths: whole 128-byte lines, then every remainder of 16 bytes, read line by line (N = 528: one tile per
+# block, 4112 and 13000: two and four tiles per wave) or, for short rows, split; M past what the row-streaming kernel takes
+@pytest.mark.parametrize("fmt", ["bf16", "fp8"])
+@pytest.mark.parametrize("N,row_bytes,M", [(528, 8192, 9), (4112, 2048, 16), (528, 8208, 16), (531, 8320 - 16, 9),
+                                           (4112, 1280 + 16, 16), (4112, 1280 + 32, 8), (4100, 4096 + 48, 11),
+                                           (4112, 2048 + 64, 9), (13000, 1408 + 80, 16), (8200, 2176 - 32, 8),
+                                           (4112, 1024 + 112, 16), (528, 1024 + 80, 12), (8200, 16, 9), (4112, 9200, 8)])
+def test_row_forms(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
+    """Also from weights 16 bytes past a line (bit for bit the same), and with a row of NaN between finite ones: rows that share
+    its lines keep their results."""
+    K = row_bytes // (2 if fmt == "bf16" else 1)
+    ops, np_ops = make(fmt, N, K, bias=True)
+    dev = to_device(ops, cuda)
+    x = x_rows(M, K, 8000 + M + N + K)
+    rows = np.unique(np.concatenate([np.arange(0, N, max(1, N // 100)), np.arange(max(0, N - 17), N)])).astype(np.int64)
+    refs = oracle_rows(oracle, fmt, np_ops, xbits(x), rows)
+    note(f"tile row forms {fmt} M={M} N={N} row bytes {row_bytes}")
+    x = x.to(cuda)
+    y = run_batch(gemv_lib, fmt, dev, x)
+    torch.cuda.synchronize()
+    check_rows(oracle, y, refs, f"tile {fmt} M={M} {N}x{K}", rows)
+    name = "W" if fmt == "bf16" else "Wq"
+    w = dev[name].contiguous().view(torch.uint8).view(-1)
+    room = torch.empty(w.numel() + 16, dtype=torch.uint8, device=cuda)
+    room[16:].copy_(w)
+    moved = dict(dev)
+    moved[name] = room[16:].view(dev[name].dtype).view(dev[name].shape)
+    y2 = run_batch(gemv_lib, fmt, moved, x)
+    torch.cuda.synchronize()
+    assert torch.equal(y2.view(torch.int16), y.view(torch.int16))
+    bad = torch.arange(5, N, 7, device=cuda)
+    room[16:].view(N, row_bytes)[bad] = 0x7F if fmt == "fp8" else 0xFF   # e4m3 and bf16 NaN
+    y3 = run_batch(gemv_lib, fmt, moved, x)
+    torch.cuda.synchronize()
+    assert torch.isnan(y3[:, bad]).all()
+    keep = torch.ones(N, dtype=torch.bool, device=cuda)
+    keep[bad] = False
+    assert torch.equal(y3[:, keep].view(torch.int16), y[:, keep].view(torch.int16))
