@@ -261,9 +261,10 @@ int pick(int kind, int M, int N, int K)
 //   * at most 128 tiles, where a block per tile leaves half the CUs idle: FP8 1000x3584 M = 2 3.22 / 3.86, M = 4 3.76 /
 //     4.12; BF16 M = 4 4.30 / 5.25, M = 7 and 8 even; INT4 M = 2 3.48 / 4.2, M = 3 even;
 //   * up to 1024 tiles of ordinary K, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even), FP8 M = 2
-//     (6144x4096 6.51 / 7.10, 10112x4096 9.19 / 10.09; M = 3 7.54 / 7.23), INT4 M = 2 up to 256 tiles (4096x4096 4.84 / 5.2, 1455x1920 3.31 / 3.64, 3000x1536 4.44 / 3.31;
-//     6144x4096 even), and the same at any N for K up to 2560 (BF16 33000x2048 M = 2 21.5 / 22.4); and BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 / 29.4, M = 5 29.2 /
-//     30.7). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
+//     (6144x4096 6.51 / 7.10, 10112x4096 9.19 / 10.09; M = 3 7.54 / 7.23), INT4 M = 2 up to 256 tiles (4096x4096
+//     4.84 / 5.2, 1455x1920 3.31 / 3.64, 3000x1536 4.44 / 3.31; 6144x4096 even), and the same at any N for K up to 2560 (BF16
+//     33000x2048 M = 2 21.5 / 22.4); and BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 /
+//     29.4, M = 5 29.2 / 30.7). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
 //     kernel's;
 //   * rows that are no multiple of 128 bytes, whose lines the tile kernel reads past their ends or carries through LDS: BF16 to
 //     M = 4 (40000x1512 21.3 / 23.9, 20000x5000 32.5 / 34.3, 60000x760 18.2 / 20.5; M = 5 34.2 / 32.8, from 2048 tiles
@@ -275,7 +276,9 @@ bool rows_ahead(int kind, int M, int N, int K)
 {
     const int ntiles = (N + kTileRows - 1) / kTileRows;
     const bool mid = K >= 2048 && K <= 8192;
-    if (kind >= 2) return M == 2 && ((ntiles <= 256 && K > 1536 && K <= 8192) || (ntiles > 768 && K > 8192) || (ntiles > 4096 && K >= 4096));
+    if (kind >= 2)
+        return M == 2 && ((ntiles <= 256 && K > 1536 && K <= 8192) || (ntiles > 768 && K > 8192) ||
+                          (ntiles > 4096 && K >= 4096));
     if (ntiles <= 128) return M <= (kind == 0 ? 7 : 4);
     if ((kind == 0 ? 2 * K : K) % 128 != 0) {
         if (K <= 8192 && M <= (kind != 0 ? 2 : (ntiles > 2048 ? 5 : 4))) return true;

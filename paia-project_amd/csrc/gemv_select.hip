@@ -95,8 +95,11 @@ int paia_gemv_pick_variant(int kind, int N, int K)
             for (const Pick& p : kTuned) {
                 if (p.kind != want || p.N <= 0 || p.K <= 0) continue;
                 const double d = std::fabs(std::log2((double)N / p.N)) + std::fabs(std::log2((double)K / p.K));
+                // only a nearer entry is looked up in the variant tables: that, not the distances, is this loop's time, spent
+                // on every call of the torch operators at an untuned shape (BF16 10111x4224 13.6 -> 2.7 us)
+                if (best >= 0 && !(d < best_d)) continue;
                 const int v = resolve(p);
-                if (v >= 0 && (best < 0 || d < best_d)) {
+                if (v >= 0) {
                     best = v;
                     best_d = d;
                 }
