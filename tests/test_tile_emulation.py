@@ -1,6 +1,7 @@
 """The tile kernel's index arithmetic (paia-project_amd/csrc/gemv_tile.h) replayed on the CPU: every tile has one unit and
 every stage one wave, the XCD order is a permutation, the metadata items divide exactly and stay in their LDS words, and the
 swizzled LDS layouts bring each lane the columns its MFMA step takes, without a bank conflict among 8 rows."""
+import numpy as np
 import pytest
 
 from test_batch_emulation import step_col
@@ -72,3 +73,41 @@ def test_lds_layouts(fmt):
             assert 8 * piece == step_col(fmt, j, h)          # x's 8 columns = the weights' of that lane group and step
     for p in range(4):                                       # 8 consecutive rows' same piece: 8 different 16-byte banks
         assert len({w_at(r, p) % 128 for r in range(8)}) == 8 and len({x_at(r, p) % 128 for r in range(8)}) == 8
+
+
+@pytest.mark.parametrize("rem", range(0, 128, 16))
+@pytest.mark.parametrize("row_bytes", [128, 1024, 1280])
+@pytest.mark.parametrize("splits", [4, 8])
+def test_ring_gives_every_stage_its_bytes(rem, row_bytes, splits):
+    """Rows of any 16-byte remainder read line by line: the line a lane loads, where it puts it in the two-line ring and where
+    a stage reads it, as the kernel computes them, give each stage its own 128 bytes of the row (zero past the row's end),
+    from offsets inside the tile, with the 16 rows' pieces in 16 different bank groups."""
+    rb = row_bytes + rem
+    rng = np.random.default_rng(rb)
+    tile = rng.integers(1, 256, 16 * rb, dtype=np.uint8)
+    stages = -(-rb // 128)
+    for split in range(splits):
+        k0 = split * stages // splits
+        n = (split + 1) * stages // splits - k0
+        ring = np.zeros((16, 16, 16), np.uint8)           # row, piece, byte
+        for t in range(n + 1 if n else 0):
+            for lane in range(64):
+                piece, r8 = lane % 8, lane // 8
+                ws = (r8 * rb) & 127
+                kb = k0 + t - 1
+                inside = piece * 16 - ws < rb - (kb + 1) * 128
+                off = r8 * rb - ws + piece * 16 + (kb + 1) * 128
+                for i in range(2):
+                    at = off + 8 * rb * i
+                    assert not inside or 0 <= at <= 16 * rb - 16
+                    put = (piece + r8 - (ws >> 4) + 8 * i + 8 * (t & 1)) & 15
+                    ring[8 * i + r8, put] = tile[at:at + 16] if inside else 0
+            if t == 0:
+                continue
+            for q in range(8):
+                gets = [(q + row + 8 * ((t + 1) & 1)) & 15 for row in range(16)]
+                assert len(set(gets)) == 16
+                for row in range(16):
+                    lo = (k0 + t - 1) * 128 + q * 16
+                    want = tile[row * rb + lo:row * rb + lo + 16] if lo < rb else np.zeros(16, np.uint8)
+                    assert np.array_equal(ring[row, gets[row]], want), (split, t, row, q)
