@@ -217,7 +217,8 @@ class GemvLib:
         return self.KERNELS[k]
 
     def batch_pick_variant(self, kind, M, N, K):
-        """The library's default small-batch variant (an index of variants_batch[kind]); -1 if M is out of range."""
+        """The best entry of variants_batch[kind] for the shape; -1 if M is out of range. A call whose variant is left to
+        the library may instead run the tile kernel, which has no entry."""
         return self._lib.paia_gemv_batch_pick_variant(KINDS[kind], M, N, K)
 
     def batch_bf16(self, W_ptr, x_ptr, bias_ptr, y_ptr, M, N, K, variant=-1, stream=None):
