@@ -30,13 +30,17 @@ constexpr int kShortK = 2560, kLongBf16K = 4096;
 // cache (nt fetched 1.6 times the weights' bytes: BF16 45653x10952 M = 11 250 us, plain in turn 204, RING 155; FP8
 // 72800x7024 M = 16 152 / 119 / 100). Several tiles per wave: down to 1280-byte rows (BF16 21595x664 M = 16 9.5 RING, 10.3
 // plain; 30000x520 12.2 / 10.7). One tile, which waits on latency more than it streams: K >= 4096 and more than 32 tiles
-// (FP8 4000x4944 M = 16 8.6 / 8.8, 1000x3600 6.5 / 4.8; BF16 600x18936 M = 8 22.9 / 28.0, 50x15016 M = 11 20.6 / 14.9).
+// (FP8 4000x4944 M = 16 8.6 / 8.8, 1000x3600 6.5 / 4.8; BF16 600x18936 M = 8 22.9 / 28.0, 50x15016 M = 11 20.6 / 14.9), BF16
+// from 2400-byte rows on more than 64 tiles (4000x2840 M = 8 6.5 / 7.2, 4090x1208 M = 16 4.9 / 5.3, 1207x2840 7.1 / 7.4, but
+// 900x2504 6.4 / 5.2, 700x3592 8.1 / 6.2).
 enum { kLines, kRing, kSplit };
-template <int P>
+template <int F, int P>
 int row_form(const BatchParams& b)
 {
     if (b.row_bytes % 128 == 0) return kLines;
-    return (P == 1 ? b.K >= 4096 && b.N > 32 * kTileRows : b.row_bytes >= 1280) ? kRing : kSplit;
+    if (P > 1) return b.row_bytes >= 1280 ? kRing : kSplit;
+    if (F == kBF16 && b.row_bytes >= 2400 && b.N > 64 * kTileRows) return kRing;
+    return b.K >= 4096 && b.N > 32 * kTileRows ? kRing : kSplit;
 }
 
 template <int F, int MT, int P, int W, int D>
@@ -45,7 +49,7 @@ int launch_d(const BatchParams& b, int blocks, hipStream_t st)
     if constexpr (TileFmt<F>::kI4F) {
         return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);
     } else {
-        switch (row_form<P>(b)) {
+        switch (row_form<F, P>(b)) {
         case kLines: return launch_tile<F, P, W, W, D, MT, 2, P == 1, false>(b, blocks, st);
         case kRing: return launch_tile<F, P, W, W, D, MT, 2, false, true>(b, blocks, st);
         default: return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);

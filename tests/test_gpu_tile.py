@@ -115,7 +115,7 @@ def test_int4_extreme_x(oracle, gemv_lib, cuda, fmt, lo, hi):
 @pytest.mark.parametrize("N,row_bytes,M", [(528, 8192, 9), (4112, 2048, 16), (528, 8208, 16), (531, 8320 - 16, 9),
                                            (4112, 1280 + 16, 16), (4112, 1280 + 32, 8), (4100, 4096 + 48, 11),
                                            (4112, 2048 + 64, 9), (13000, 1408 + 80, 16), (8200, 2176 - 32, 8),
-                                           (4112, 1024 + 112, 16), (528, 1024 + 80, 12), (8200, 16, 9), (4112, 9200, 8)])
+                                           (4112, 1024 + 112, 16), (528, 1024 + 80, 12), (1041, 2400 + 16, 9), (8200, 16, 9), (4112, 9200, 8)])
 def test_row_forms(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
     """Also from weights 16 bytes past a line (bit for bit the same), and with a row of NaN between finite ones: rows that share
     its lines keep their results."""
