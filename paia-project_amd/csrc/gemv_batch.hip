@@ -268,8 +268,8 @@ int pick(int kind, int M, int N, int K)
 //     kernel's;
 //   * rows that are no multiple of 128 bytes, whose lines the tile kernel reads past their ends or carries through LDS: BF16 to
 //     M = 4 (40000x1512 21.3 / 23.9, 20000x5000 32.5 / 34.3, 60000x760 18.2 / 20.5; M = 5 34.2 / 32.8; above 2048 tiles and at
-//     any K to M = 6: 40408x2592 M = 5 34.4 / 36.5, 69979x2864 M = 6 66.8 / 70.7, 37492x13336 M = 4 146 / 158), FP8 M = 2 (40000x1520 12.9 / 15.0, 40000x3008 21.1 / 22.1; M = 3 23.1 / 22.6), while
-//     K <= 8192; beyond, BF16 at one to two tiles per CU to M = 6 (5000x12008 23.2 / 26.7);
+//     any K to M = 6: 40408x2592 M = 5 34.4 / 36.5, 69979x2864 M = 6 66.8 / 70.7, 37492x13336 M = 4 146 / 158),
+//     FP8 M = 2 (40000x1520 12.9 / 15.0, 40000x3008 21.1 / 22.1; M = 3 23.1 / 22.6), while K <= 8192; beyond, BF16 at one to two tiles per CU to M = 6 (5000x12008 23.2 / 26.7);
 //   * INT4 M = 2 with long rows on many tiles (30000x14336 43.0 / 49.9, 15000x11008 20.1 / 22.0; 10000x14336 even,
 //     4096x14336 10.6 / 9.1) or a great many of ordinary K (100000x4096 44.4 / 45.7, 70000x7168 53.3 / 55.2; 60000x1920 even).
 bool rows_ahead(int kind, int M, int N, int K)
