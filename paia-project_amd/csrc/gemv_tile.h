@@ -91,17 +91,27 @@ __device__ __forceinline__ void wave_lds_order()
 }
 
 // INT4: the 128 terms of a group, up to 15 |x| each, could leave fp32's range where |x| reaches 2^116 although the output
-// (scales are small) does not. So nibbles and sums of x carry a factor 2^-11, taken back once from the finished sums: no
-// finite x overflows, and at the other end products of the smallest normal x (2^-137) are subnormals that the matrix cores
-// keep, 2^-149 apart.
-constexpr float kI4Scale = 0.25f, kI4Back = 2048.0f;   // q 2^-9 as e4m3, times 2^-2
+// (scales are small) does not. So nibbles and sums of x carry a factor 2^-11: no finite x overflows, and at the other end
+// nothing is lost (a bf16 x is a multiple of 2^-133, its products of 2^-144, and the matrix cores keep subnormals down to
+// 2^-149). The scales carry 2^4 of it back, and the finished sums the rest: sums over the groups have 2^7 of room beyond
+// fp32's range, and steps of 2^-142 where the smallest outputs are 2^-133 apart (with all 2^11 left to the end the steps
+// were 2^-138, and outputs below 2^-126 had 5% more error). An asymmetric scale that does not take the 2^4 (2^124 or more)
+// is kept as it is, with the 2^4 on its nibbles and zero point instead.
+constexpr uint32_t kI4Exp = 125, kI4ExpBig = 129;      // factor on q 2^-9 as e4m3, as a float's exponent: 2^-2, 2^2
 constexpr uint32_t kI4Ones = 0x3A003A00u;              // a bf16 pair of 2^-11
+constexpr float kI4Up = 16.0f, kI4Back = 128.0f, kF32Max = 3.4028234e38f;
 
-// e4m3 byte pair HI of w (0..15 each) -> the two integers times 2^-11, as bf16
+// Metadata word of an asymmetric group (scale bf16 in the upper half of `s`): scale, exponent of the nibbles' factor, zero
+// point. The scale's 2^4 is exact in bf16, also for a subnormal one.
+__device__ __forceinline__ uint32_t i4zp_word(float up, uint32_t z) { return __float_as_uint(up) | kI4Exp << 8 | z; }
+__device__ __forceinline__ uint32_t i4zp_word_big(uint32_t s, uint32_t z) { return s | kI4ExpBig << 8 | z << 4; }
+
+// e4m3 byte pair HI of w (0..15 each) -> the two integers times 2^-9 and the scale's power of two (the conversion takes the
+// exponent field of `scale` only), as bf16
 template <bool HI>
-__device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w)
+__device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w, float scale)
 {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, kI4Scale, HI));
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, HI));
 }
 
 // P tiles per unit, S waves sharing them along K (W / S units per block), D stages in flight per wave, MT activation
@@ -177,10 +187,24 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     uint32_t* md = reinterpret_cast<uint32_t*>(smem);
     auto meta_put = [&](int i, const Meta& m) {
         const uint32_t r = __umulhi((uint32_t)i, p.chunk_mul), c = (uint32_t)i - r * (uint32_t)p.chunks;
+        uint32_t* at = md + 4u * c * (uint32_t)p.mstride + r;
+        uint32_t s[4];
+        float up[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const uint32_t sv = g & 1 ? m.s[g >> 1] & 0xFFFF0000u : m.s[g >> 1] << 16;
-            md[(4u * c + (uint32_t)g) * (uint32_t)p.mstride + r] = sv | ((m.z >> (4 * g)) & 15u);
+            s[g] = g & 1 ? m.s[g >> 1] & 0xFFFF0000u : m.s[g >> 1] << 16;
+            up[g] = (F == kI4 ? f16_to_f32(s[g] >> 16) : __uint_as_float(s[g])) * kI4Up;
+            at[(uint32_t)g * (uint32_t)p.mstride] =
+                F == kI4 ? __float_as_uint(up[g]) : i4zp_word(up[g], (m.z >> (4 * g)) & 15u);
+        }
+        if constexpr (F == kI4ZP) {   // a branch hardly ever taken: chosen word by word it cost 0.07 us a launch more
+            const float top = fmaxf(fmaxf(fabsf(up[0]), fabsf(up[1])), fmaxf(fabsf(up[2]), fabsf(up[3])));
+            if (__builtin_expect(top > kF32Max, 0)) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    if (fabsf(up[g]) > kF32Max)
+                        at[(uint32_t)g * (uint32_t)p.mstride] = i4zp_word_big(s[g], (m.z >> (4 * g)) & 15u);
+            }
         }
     };
     Meta m0;
@@ -322,6 +346,8 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
 #pragma unroll
         for (int t2 = 0; t2 < P; ++t2) {
             u32x4 w[L];
+            uint32_t m = 0u;   // INT4: read ahead of the weights, whose decode needs it
+            if constexpr (I4) m = mw[(uint32_t)kb * (uint32_t)p.mstride + (uint32_t)(t2 * kTileRows)];
             if (t2 >= kSlots) wave_lds_order();
 #pragma unroll
             for (int i = 0; i < L; ++i) w[i] = get_w(t2, i, t);
@@ -340,16 +366,16 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
                                                fp8x2_to_bf16x2<false>(d1), fp8x2_to_bf16x2<true>(d1)}, acc[t2]);
                 }
             } else {
+                const float f = __uint_as_float(F == kI4 ? kI4Exp << 23 : m << 15);   // bits 8..15 to the exponent
                 f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < X; ++j) {
                     const uint32_t v = j == 0 ? w[0].x : (j == 1 ? w[0].y : (j == 2 ? w[0].z : w[0].w));
                     const uint32_t lo = v & 0x0F0F0F0Fu, hi = (v >> 4) & 0x0F0F0F0Fu;
-                    g = mfma(a[j], u32x4{i4x2_to_bf16x2<false>(lo), i4x2_to_bf16x2<true>(lo),
-                                         i4x2_to_bf16x2<false>(hi), i4x2_to_bf16x2<true>(hi)}, g);
+                    g = mfma(a[j], u32x4{i4x2_to_bf16x2<false>(lo, f), i4x2_to_bf16x2<true>(lo, f),
+                                         i4x2_to_bf16x2<false>(hi, f), i4x2_to_bf16x2<true>(hi, f)}, g);
                 }
-                const uint32_t m = mw[(uint32_t)kb * (uint32_t)p.mstride + (uint32_t)(t2 * kTileRows)];
-                const float s = F == kI4 ? f16_to_f32(m >> 16) : __uint_as_float(m & 0xFFFF0000u);
+                const float s = __uint_as_float(F == kI4 ? m : m & 0xFFFF0000u);
                 const float z = F == kI4 ? 8.0f : (float)(m & 0xFFu);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) acc[t2][v] = __builtin_fmaf(s, __builtin_fmaf(-z, xs[v], g[v]), acc[t2][v]);

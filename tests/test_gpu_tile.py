@@ -109,6 +109,48 @@ def test_int4_extreme_x(oracle, gemv_lib, cuda, fmt, lo, hi):
         assert np.abs(got - r64).max() / np.abs(r64).max() < 2e-2, m
 
 
+@pytest.mark.parametrize("fmt", ["int4", "int4zp"])
+@pytest.mark.parametrize("M", [5, 16])
+def test_int4_smallest_outputs(oracle, gemv_lib, cuda, fmt, M):
+    """Outputs in bf16's subnormal range carry the error of their rounding and no more. The fp32 sums move in steps of 2^-142
+    there: over the 32 groups of K = 4096 that adds 32 / 12 * 2^-284 to the rounding's variance 2^-266 / 12, a relative 1.2e-4
+    (sums in steps of 2^-138 would add 3%)."""
+    N, K = 2064, 4096
+    ops, np_ops = make(fmt, N, K)
+    x = (x_rows(M, K, 31).double() * 2.0 ** -129).to(torch.bfloat16)
+    note(f"tile smallest outputs {fmt} M={M}")
+    y = run_batch(gemv_lib, fmt, to_device(ops, cuda), x.to(cuda)).float().cpu().numpy().astype(np.float64)
+    want = np.stack([r for r, _ in oracle_rows(oracle, fmt, np_ops, xbits(x))])
+    assert 2.0 ** -130 < np.sqrt((want ** 2).mean()) and np.abs(want).max() < 2.0 ** -125
+    rounding = np.rint(want * 2.0 ** 133) * 2.0 ** -133 - want
+    assert np.sqrt(((y - want) ** 2).mean() / (rounding ** 2).mean()) < 1.005
+
+
+def test_int4zp_largest_scales(oracle, gemv_lib, cuda):
+    """One group with a scale of 2^124: its row is right, and every other row of the call keeps its bits. An infinite scale
+    stays in its row too."""
+    N, K, M = 4112, 1024, 6
+    ops, np_ops = make("int4zp", N, K)
+    dev = to_device(ops, cuda)
+    x = (x_rows(M, K, 32).double() * 2.0 ** -12).to(torch.bfloat16)
+    xd = x.to(cuda)
+    note("tile largest scales int4zp")
+    want = run_batch(gemv_lib, "int4zp", dev, xd)
+    scales = ops["scales"].clone()
+    scales[100, 3] = 2.0 ** 124
+    big = dict(dev, scales=scales.to(cuda))
+    y = run_batch(gemv_lib, "int4zp", big, xd)
+    np_big = dict(np_ops, scales=scales.view(torch.int16).numpy().view(np.uint16))
+    rows = np.array([100], dtype=np.int64)
+    check_rows(oracle, y, oracle_rows(oracle, "int4zp", np_big, xbits(x), rows), "row 100", rows)
+    keep = torch.arange(N, device=cuda) != 100
+    assert torch.equal(y[:, keep].view(torch.int16), want[:, keep].view(torch.int16))
+    scales[100, 3] = float("inf")
+    y = run_batch(gemv_lib, "int4zp", dict(dev, scales=scales.to(cuda)), xd)
+    assert not torch.isfinite(y[:, 100]).any()
+    assert torch.equal(y[:, keep].view(torch.int16), want[:, keep].view(torch.int16))
+
+
 # BF16 and FP8 row lengths: whole 128-byte lines, then every remainder of 16 bytes, read line by line (N = 528: one tile per
 # block, 4112 and 13000: two and four tiles per wave) or, for short rows, split; M past what the row-streaming kernel takes
 @pytest.mark.parametrize("fmt", ["bf16", "fp8"])

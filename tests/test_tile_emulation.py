@@ -1,6 +1,7 @@
 """The tile kernel's index arithmetic (paia-project_amd/csrc/gemv_tile.h) replayed on the CPU: every tile has one unit and
 every stage one wave, the XCD order is a permutation, the metadata items divide exactly and stay in their LDS words, and the
-swizzled LDS layouts bring each lane the columns its MFMA step takes, without a bank conflict among 8 rows."""
+swizzled LDS layouts bring each lane the columns its MFMA step takes, without a bank conflict among 8 rows. Also its INT4
+decode: nibbles as e4m3 bytes, their pairs against the re-paired activations, and the powers of two on the way."""
 import numpy as np
 import pytest
 
@@ -111,3 +112,46 @@ def test_ring_gives_every_stage_its_bytes(rem, row_bytes, splits):
                     lo = (k0 + t - 1) * 128 + q * 16
                     want = tile[row * rb + lo:row * rb + lo + 16] if lo < rb else np.zeros(16, np.uint8)
                     assert np.array_equal(ring[row, gets[row]], want), (split, t, row, q)
+
+
+def e4m3(b):                                              # codes 0..15: subnormals and the first binade
+    return b * 2.0 ** -9 if b < 8 else (1 + (b - 8) / 8) * 2.0 ** -6
+
+
+def test_int4_nibbles_as_e4m3():
+    """All 16 codes in every position of a word: the byte pairs taken as e4m3, times 2^-2, are q 2^-11 in the order in which
+    the activations are re-paired, so that a group's products are its weights' own."""
+    order = [0, 2, 4, 6, 1, 3, 5, 7]                      # columns of a step's four bf16 pairs (i4_pair_x)
+    perm = lambda hi, lo, sel: [(lo + hi)[k] for k in sel]
+    x = np.arange(8)
+    pairs = [x[0:2].tolist(), x[2:4].tolist(), x[4:6].tolist(), x[6:8].tolist()]
+    paired = (perm(pairs[1], pairs[0], [0, 2]) + perm(pairs[3], pairs[2], [0, 2]) +
+              perm(pairs[1], pairs[0], [1, 3]) + perm(pairs[3], pairs[2], [1, 3]))
+    assert paired == order
+    for word in [int("".join(f"{(q + 5 * j) % 16:x}" for j in range(8)), 16) for q in range(16)]:
+        lo, hi = word & 0x0F0F0F0F, (word >> 4) & 0x0F0F0F0F
+        got = [e4m3((h >> (8 * b)) & 0xFF) * 0.25 for h in (lo, hi) for b in range(4)]
+        assert got == [((word >> (4 * c)) & 15) * 2.0 ** -11 for c in order]
+
+
+def test_int4_powers_of_two():
+    """Nibbles and sums of x at 2^-11, scales at 2^4, the finished sums times 2^7: the powers cancel, no group of finite
+    activations leaves fp32, and products of the smallest activations are exact in it. Asymmetric scales keep every bit in
+    the metadata word, those too large for the 2^4 with it on the nibbles and the zero point."""
+    f32max, xmax, xmin = (2 - 2.0 ** -23) * 2.0 ** 127, (2 - 2.0 ** -7) * 2.0 ** 127, 2.0 ** -133
+    assert np.array([0x3A00 << 16], np.uint32).view(np.float32)[0] == 2.0 ** -11
+    assert 128 * 15 * 2.0 ** -11 * xmax < f32max and xmin * 2.0 ** -11 >= 2.0 ** -149
+    s16 = np.arange(1 << 16, dtype=np.uint32)             # every bf16
+    s16 = s16[(s16 & 0x7F80) != 0x7F80]
+    s = (s16 << 16).view(np.float32).astype(np.float64)
+    big = (s16 & 0x7F80) >= 0x7D80
+    with np.errstate(over="ignore"):
+        up = ((s16 << 16).view(np.float32) * np.float32(16)).view(np.uint32)
+    assert not np.any(up[~big] & 0xFFFF)
+    for z in (0, 5, 15):
+        word = np.where(big, s16 << 16 | 129 << 8 | z << 4, up | 125 << 8 | z)
+        scale = (word & 0xFFFF0000).astype(np.uint32).view(np.float32).astype(np.float64)
+        factor = 2.0 ** (((word << 15 >> 23) & 0xFF).astype(np.int64) - 127)
+        assert np.isfinite(scale).all()
+        assert np.array_equal(scale * factor * 2.0 ** -9 * 2.0 ** 7, s)                      # on the nibbles
+        assert np.array_equal(scale * (word & 0xFF) * 2.0 ** -11 * 2.0 ** 7, s * z)          # on the sums of x
