@@ -24,6 +24,7 @@ namespace {
 //   * The stages go to the waves in turn for one tile per wave and for INT4 (28672x4096 M = 4 15.8, 17.1 in contiguous
 //     ranges), in contiguous ranges otherwise (FP8 14336x4096 M = 16 12.6, 13.3 in turn).
 constexpr int kShortK = 2560, kLongBf16K = 4096;
+constexpr int kTileMaxRows = (1 << 30) - (1 << 16);
 
 // Rows that are no multiple of 128 bytes (BF16, FP8): every stage's bytes of a row lie in two lines. Read line by line where
 // a wave's range pays for its extra line (RING); else plain loads in turn, so that the second stage of a line finds it in
@@ -122,8 +123,9 @@ int launch_fmt(const BatchParams& b, hipStream_t st)
 
 int launch_tile_picked(int kind, const BatchParams& b, hipStream_t st)
 {
-    // the kernel's index arithmetic: rows in 31 bits, a tile's weights and x behind one 31-bit buffer offset
-    if (b.M < 2 || b.M > kMaxBatch || b.N > (1 << 30) || b.K > (1 << 24)) return kTileRefused;
+    // the kernel's index arithmetic: rows in 31 bits, N * 4 bytes of FP8 scales and a launch's threads (at least 64 rows per
+    // 256, N this large leaves room for short rows only) in 32, a tile's weights and x behind one 31-bit buffer offset
+    if (b.M < 2 || b.M > kMaxBatch || b.N > kTileMaxRows || b.K > (1 << 24)) return kTileRefused;
     switch (kind) {
     case 0: return launch_fmt<kBF16>(b, st);
     case 1: return launch_fmt<kFP8>(b, st);

@@ -2,6 +2,9 @@
 every stage one wave, the XCD order is a permutation, the metadata items divide exactly and stay in their LDS words, and the
 swizzled LDS layouts bring each lane the columns its MFMA step takes, without a bank conflict among 8 rows. Also its INT4
 decode: nibbles as e4m3 bytes, their pairs against the re-paired activations, and the powers of two on the way."""
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -19,6 +22,21 @@ def test_tiles_and_blocks(tiles, blocks, units):
     order = [(x * (per + 1) if x < rem else rem * (per + 1) + (x - rem) * per) + b // 8
              for b in range(blocks) for x in [b % 8]]
     assert sorted(order) == list(range(blocks))
+
+
+def test_most_rows():
+    """At the most rows the launch takes (short rows: rounds of three blocks of 256 threads per CU, at most four tiles each),
+    fewer than 2^32 threads and FP8 scales within a 32-bit buffer size."""
+    src = (Path(__file__).resolve().parent.parent / "paia-project_amd/csrc/gemv_tile.hip").read_text()
+    most = eval(re.search(r"kTileMaxRows = (.*);", src).group(1))
+    assert most * 4 < 1 << 32
+    for cus in (32, 128, 256, 304):
+        for N in [most - d for d in (0, 1, 15, 16, 17, 12288, 1 << 20)] + [1 << 29, 1 << 28]:
+            ntiles = -(-N // 16)
+            blocks = 3 * cus * -(-ntiles // (12 * cus))
+            P = -(-ntiles // blocks)
+            fewest = -(-ntiles // P)
+            assert P <= 4 and max(blocks, fewest) * 256 < 1 << 32
 
 
 @pytest.mark.parametrize("stages", [1, 3, 4, 7, 28, 32, 147, 148, 300])
