@@ -109,8 +109,9 @@ __global__ void __launch_bounds__(T < 256 ? 256 : T) quantize_fp8_kernel(const f
     const float s = amax > 0.0f ? amax / 448.0f : 1.0f;
     if (tid == 0) scale[n] = s;
     uint32_t* qrow = reinterpret_cast<uint32_t*>(q + (size_t)n * K);
-    const bool fast = div_by_ok(s);
-    const float y = 1.0f / s;
+    constexpr bool kFew = KEEP && V == 1;          // four quotients: the reciprocal would only lengthen the chain
+    const bool fast = !kFew && div_by_ok(s);
+    const float y = kFew ? 0.0f : 1.0f / s;
     auto code = [&](const f32x4v a) -> uint32_t {
         auto c = [&](float w) {
             const float t = fast ? div_by(w, s, y) : w / s;
@@ -127,9 +128,10 @@ __global__ void __launch_bounds__(T < 256 ? 256 : T) quantize_fp8_kernel(const f
     }
 }
 
-// ---- INT4: 16 lanes per group, kQSteps x 4 groups per wave -----------------------------------------------------------
+// ---- INT4: L lanes per group, `Steps` steps of 64 / L groups per wave -------------------------------------------------
+// Many groups: 16 lanes of 8 weights, two steps. Few: the lanes' chain of quotients is the call's time, so 64 lanes of two
+// weights (asymmetric 32 of four, a pair of groups per wave).
 constexpr int kQBlock = 256;
-constexpr int kQSteps = 2;
 
 __device__ __forceinline__ float row16_max(float v)   // over the 16 lanes of a DPP row, in every lane of it
 {
@@ -138,79 +140,123 @@ __device__ __forceinline__ float row16_max(float v)   // over the 16 lanes of a 
     v = fmaxf(v, dpp_f32<0x124>(v));
     return fmaxf(v, dpp_f32<0x128>(v));
 }
-struct Group8 {
-    float w[8];
-};
-__device__ __forceinline__ Group8 group_load(const float* W, size_t gi, int l16, bool ok)
+template <int L>
+__device__ __forceinline__ float group_max(float v)
 {
-    f32x4v a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
-    if (ok) {
-        const float* p = W + gi * 128 + (size_t)(l16 * 8);
-        a = ld4(p);
-        b = ld4(p + 4);
+    if constexpr (L == 64) return wave_max(v);
+    v = row16_max(v);
+    if constexpr (L == 32) {
+        const int b = __float_as_int(v);
+        const float lo = fmaxf(v, __int_as_float(__builtin_amdgcn_readlane(b, 16)));   // rows 0, 1 (valid in row 0)
+        const float hi = fmaxf(v, __int_as_float(__builtin_amdgcn_readlane(b, 48)));   // rows 2, 3 (valid in row 2)
+        const int l = __builtin_amdgcn_readlane(__float_as_int(lo), 0), h = __builtin_amdgcn_readlane(__float_as_int(hi), 32);
+        v = __int_as_float(lane_id() < 32 ? l : h);
     }
-    return {{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+    return v;
 }
-// The 8 codes of a lane as one word (weight j in nibble j).
-template <bool ZP>
-__device__ __forceinline__ uint32_t group_codes(const Group8& g, float s, float z)
+template <int L>
+struct GroupPart {
+    float w[128 / L];
+};
+template <int L>
+__device__ __forceinline__ GroupPart<L> group_load(const float* W, size_t gi, int l, bool ok)
 {
-    const bool fast = div_by_ok(s);
-    const float y = 1.0f / s;
+    constexpr int n = 128 / L;
+    GroupPart<L> g;
+#pragma unroll
+    for (int j = 0; j < n; ++j) g.w[j] = 0.0f;
+    if (ok) {
+        const float* p = W + gi * 128 + (size_t)(l * n);
+        if constexpr (n == 2) {
+            const float2 a = *reinterpret_cast<const float2*>(p);
+            g.w[0] = a.x;
+            g.w[1] = a.y;
+        } else {
+#pragma unroll
+            for (int j = 0; j < n; j += 4) {
+                const f32x4v a = ld4(p + j);
+                g.w[j] = a.x;
+                g.w[j + 1] = a.y;
+                g.w[j + 2] = a.z;
+                g.w[j + 3] = a.w;
+            }
+        }
+    }
+    return g;
+}
+// The codes of a lane as one word (weight j in nibble j).
+template <bool ZP, int L>
+__device__ __forceinline__ uint32_t group_codes(const GroupPart<L>& g, float s, float z)
+{
+    constexpr bool kFew = L > 16;   // few quotients: the reciprocal would only lengthen the chain
+    const bool fast = !kFew && div_by_ok(s);
+    const float y = kFew ? 0.0f : 1.0f / s;
     uint32_t word = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 128 / L; ++j) {
         const float t = __builtin_rintf(fast ? div_by(g.w[j], s, y) : g.w[j] / s);
         const int c = ZP ? (int)fminf(fmaxf(t + z, 0.0f), 15.0f) : (int)fminf(fmaxf(t, -7.0f), 7.0f) + 8;
         word |= (uint32_t)c << (4 * j);
     }
     return word;
 }
+template <int L>
+__device__ __forceinline__ void group_store(uint8_t* packed, size_t gi, int l, uint32_t word)
+{
+    uint8_t* p = packed + gi * 64 + (size_t)(l * (64 / L));
+    if constexpr (L == 16) *reinterpret_cast<uint32_t*>(p) = word;
+    else if constexpr (L == 32) *reinterpret_cast<uint16_t*>(p) = (uint16_t)word;
+    else *p = (uint8_t)word;
+}
 
+template <int L, int Steps>
 __global__ void __launch_bounds__(kQBlock) quantize_int4_kernel(const float* __restrict__ W,
                                                                 uint8_t* __restrict__ packed,
                                                                 uint16_t* __restrict__ scales, size_t ngroups)
 {
-    const int lane = lane_id(), l16 = lane & 15;
-    const size_t g0 = ((size_t)blockIdx.x * (kQBlock / kWave) + (size_t)wave_id()) * (4 * kQSteps) + (size_t)(lane >> 4);
-    Group8 g[kQSteps];
+    constexpr int kPer = 64 / L;   // groups per wave and step
+    const int lane = lane_id(), l = lane % L;
+    const size_t g0 = ((size_t)blockIdx.x * (kQBlock / kWave) + (size_t)wave_id()) * (kPer * Steps) + (size_t)(lane / L);
+    GroupPart<L> g[Steps];
 #pragma unroll
-    for (int e = 0; e < kQSteps; ++e) g[e] = group_load(W, g0 + 4 * e, l16, g0 + 4 * e < ngroups);
+    for (int e = 0; e < Steps; ++e) g[e] = group_load<L>(W, g0 + kPer * e, l, g0 + kPer * e < ngroups);
 #pragma unroll
-    for (int e = 0; e < kQSteps; ++e) {
-        const size_t gi = g0 + 4 * e;
+    for (int e = 0; e < Steps; ++e) {
+        const size_t gi = g0 + kPer * e;
         float amax = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(g[e].w[j]));
-        amax = row16_max(amax);
+        for (int j = 0; j < 128 / L; ++j) amax = fmaxf(amax, fabsf(g[e].w[j]));
+        amax = group_max<L>(amax);
         const _Float16 s16 = (_Float16)(amax > 0.0f ? amax / 7.0f : 1.0f);   // v_cvt_f16_f32: round to nearest even
         float sf = (float)s16;
         if (!(sf > 0.0f)) sf = 1.0f;
-        const uint32_t word = group_codes<false>(g[e], sf, 0.0f);
+        const uint32_t word = group_codes<false, L>(g[e], sf, 0.0f);
         if (gi < ngroups) {
-            reinterpret_cast<uint32_t*>(packed)[gi * 16 + (size_t)l16] = word;
-            if (l16 == 0) scales[gi] = __builtin_bit_cast(uint16_t, s16);
+            group_store<L>(packed, gi, l, word);
+            if (l == 0) scales[gi] = __builtin_bit_cast(uint16_t, s16);
         }
     }
 }
 
-// A pair of groups (2j, 2j+1 of a row) is 32 lanes, so the packed zero-point byte has one writer: the second group's first
-// lane, or the first's where G is odd (ODD) and the pair is the row's last.
-template <bool ODD>
+// A pair of groups (2j, 2j+1 of a row) is 2 L lanes of a wave, so the packed zero-point byte has one writer: the second
+// group's first lane, or the first's where G is odd (ODD) and the pair is the row's last.
+template <bool ODD, int L, int Steps>
 __global__ void __launch_bounds__(kQBlock) quantize_int4_zp_kernel(const float* __restrict__ W,
                                                                    uint8_t* __restrict__ packed,
                                                                    uint16_t* __restrict__ scales,
                                                                    uint8_t* __restrict__ zeros, uint32_t npairs, int G)
 {
-    const int lane = lane_id(), l16 = lane & 15, h = (lane >> 4) & 1;
-    const uint32_t p0 = (blockIdx.x * (kQBlock / kWave) + (uint32_t)wave_id()) * (2 * kQSteps) + (uint32_t)(lane >> 5);
+    static_assert(L == 16 || L == 32, "a pair within a wave");
+    constexpr int kPer = 32 / L;   // pairs per wave and step
+    const int lane = lane_id(), l = lane % L, h = (lane / L) & 1;
+    const uint32_t p0 = (blockIdx.x * (kQBlock / kWave) + (uint32_t)wave_id()) * (kPer * Steps) + (uint32_t)(lane / (2 * L));
     const uint32_t ZB = (uint32_t)(G + 1) / 2;
-    Group8 g[kQSteps];
-    size_t gis[kQSteps];
-    bool ok[kQSteps], alone[kQSteps];
+    GroupPart<L> g[Steps];
+    size_t gis[Steps];
+    bool ok[Steps], alone[Steps];
 #pragma unroll
-    for (int e = 0; e < kQSteps; ++e) {
-        const uint32_t pi = p0 + 2 * e;
+    for (int e = 0; e < Steps; ++e) {
+        const uint32_t pi = p0 + kPer * e;
         alone[e] = false;
         ok[e] = pi < npairs;
         if constexpr (ODD) {
@@ -221,18 +267,18 @@ __global__ void __launch_bounds__(kQBlock) quantize_int4_zp_kernel(const float* 
         } else {
             gis[e] = 2 * (size_t)pi + (size_t)h;
         }
-        g[e] = group_load(W, gis[e], l16, ok[e]);
+        g[e] = group_load<L>(W, gis[e], l, ok[e]);
     }
 #pragma unroll
-    for (int e = 0; e < kQSteps; ++e) {
+    for (int e = 0; e < Steps; ++e) {
         float lo = g[e].w[0], hi = g[e].w[0];
 #pragma unroll
-        for (int j = 1; j < 8; ++j) {
+        for (int j = 1; j < 128 / L; ++j) {
             lo = fminf(lo, g[e].w[j]);
             hi = fmaxf(hi, g[e].w[j]);
         }
-        lo = fminf(-row16_max(-lo), 0.0f);
-        hi = fmaxf(row16_max(hi), 0.0f);
+        lo = fminf(-group_max<L>(-lo), 0.0f);
+        hi = fmaxf(group_max<L>(hi), 0.0f);
         const float r = (hi - lo) / 15.0f;
         uint32_t sb = f32_to_bf16_rne(r);
         float s = bf16_to_f32(sb);
@@ -241,16 +287,17 @@ __global__ void __launch_bounds__(kQBlock) quantize_int4_zp_kernel(const float* 
             s = 1.0f;
         }
         const float zf = fminf(fmaxf(__builtin_rintf(-lo / s), 0.0f), 15.0f);
-        const uint32_t word = group_codes<true>(g[e], s, zf);
-        // the first group's zero point to the second's lanes (row_bcast:15 into rows 1 and 3)
+        const uint32_t word = group_codes<true, L>(g[e], s, zf);
+        // the first group's zero point to the second's lanes (L = 16: row_bcast:15 into rows 1 and 3)
         const uint32_t z = (uint32_t)zf;
-        const uint32_t zfirst = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)z, 0x142, 0xA, 0xF, false);
+        const uint32_t zfirst = L == 16 ? (uint32_t)__builtin_amdgcn_update_dpp(0, (int)z, 0x142, 0xA, 0xF, false)
+                                        : (uint32_t)__builtin_amdgcn_readlane((int)z, 0);
         if (ok[e]) {
-            reinterpret_cast<uint32_t*>(packed)[gis[e] * 16 + (size_t)l16] = word;
-            if (l16 == 0) {
+            group_store<L>(packed, gis[e], l, word);
+            if (l == 0) {
                 scales[gis[e]] = (uint16_t)sb;
-                if (h) zeros[p0 + 2 * e] = (uint8_t)(zfirst | (z << 4));
-                else if (alone[e]) zeros[p0 + 2 * e] = (uint8_t)z;
+                if (h) zeros[p0 + kPer * e] = (uint8_t)(zfirst | (z << 4));
+                else if (alone[e]) zeros[p0 + kPer * e] = (uint8_t)z;
             }
         }
     }
@@ -287,6 +334,50 @@ int launch_fp8(const void* W, void* q, void* scale, int N, int K, hipStream_t st
     return 0;
 }
 
+template <int L, int Steps>
+int launch_int4(const void* W, void* packed, void* scales, int N, int K, hipStream_t st)
+{
+    const size_t G = (size_t)K / 128;
+    constexpr size_t kPerBlock = kQBlock / kWave * (64 / L) * Steps;
+    const size_t step = slice_rows(G, kPerBlock);
+    for (size_t n = 0; n < (size_t)N; n += step) {
+        const size_t ngroups = ((size_t)N - n < step ? (size_t)N - n : step) * G;
+        hipLaunchKernelGGL((quantize_int4_kernel<L, Steps>), dim3(blocks_for(ngroups, kPerBlock)), dim3(kQBlock), 0, st,
+                           static_cast<const float*>(W) + n * (size_t)K, static_cast<uint8_t*>(packed) + n * (size_t)(K / 2),
+                           static_cast<uint16_t*>(scales) + n * G, ngroups);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+
+template <int L, int Steps>
+int launch_int4_zp(const void* W, void* packed, void* scales, void* zeros, int N, int K, hipStream_t st)
+{
+    const size_t G = (size_t)K / 128, ZB = (G + 1) / 2;
+    constexpr size_t kPerBlock = kQBlock / kWave * (32 / L) * Steps;
+    const size_t step = slice_rows(ZB, kPerBlock);
+    for (size_t n = 0; n < (size_t)N; n += step) {
+        const size_t pairs = ((size_t)N - n < step ? (size_t)N - n : step) * ZB;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks_for(pairs, kPerBlock)), dim3(kQBlock), 0, st,
+                               static_cast<const float*>(W) + n * (size_t)K, static_cast<uint8_t*>(packed) + n * (size_t)(K / 2),
+                               static_cast<uint16_t*>(scales) + n * G, static_cast<uint8_t*>(zeros) + n * ZB, (uint32_t)pairs,
+                               (int)G);
+        };
+        if (G & 1) launch(quantize_int4_zp_kernel<true, L, Steps>);
+        else launch(quantize_int4_zp_kernel<false, L, Steps>);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+
+// Up to this many weights the forms with fewer weights a lane are ahead (us, few / many): FP8 rows of at most 1024, a block
+// against a wave each, 36x800 2.0 / 2.9, 653x976 3.0 / 3.2, 1057x672 even, 2765x1024 6.3 / 5.1; INT4 163x768 1.9 / 2.9,
+// 0.9 to 1.2 million weights 3.25 / 3.42, 1.75 to 2.2 million 5.5 / 4.7; asymmetric 67x1408 2.1 / 3.1, 0.55 to 0.93 million
+// 3.2 / 3.5, 1.1 to 1.8 million even.
+constexpr int64_t kFewWeights = 1 << 20;
+bool few(int N, int K) { return (int64_t)N * K <= kFewWeights; }
+
 }  // namespace
 
 extern "C" {
@@ -298,6 +389,7 @@ int paia_quantize_fp8_rowwise(const void* W, void* q, void* scale, int N, int K,
     // The fewest threads that hold the row with up to 8 float4 (32 registers) each, so that rows in flight fill the chip
     // between a row's two halves; a block for 1024 < K <= 2048, where a wave with 8 left few-row calls longer in flight
     // (513x1040 3.5 us against 3.1).
+    if (K <= 256 * 4 && few(N, K)) return launch_fp8<256, 1, true>(W, q, scale, N, K, st);
     if (K <= 64 * 4 * 4) return launch_fp8<64, 4, true>(W, q, scale, N, K, st);
     if (K <= 256 * 4 * 2) return launch_fp8<256, 2, true>(W, q, scale, N, K, st);
     if (K <= 256 * 4 * 4) return launch_fp8<256, 4, true>(W, q, scale, N, K, st);
@@ -310,18 +402,8 @@ int paia_quantize_fp8_rowwise(const void* W, void* q, void* scale, int N, int K,
 int paia_quantize_int4_g128(const void* W, void* packed, void* scales, int N, int K, void* stream)
 {
     if (N <= 0 || K <= 0 || (K & 127) || !aligned(W, 16) || !aligned(packed, 16) || !aligned(scales, 2)) return -2;
-    const size_t G = (size_t)K / 128;
-    constexpr size_t kPerBlock = kQBlock / kWave * 4 * kQSteps;
-    const size_t step = slice_rows(G, kPerBlock);
-    for (size_t n = 0; n < (size_t)N; n += step) {
-        const size_t ngroups = ((size_t)N - n < step ? (size_t)N - n : step) * G;
-        hipLaunchKernelGGL(quantize_int4_kernel, dim3(blocks_for(ngroups, kPerBlock)), dim3(kQBlock), 0,
-                           static_cast<hipStream_t>(stream), static_cast<const float*>(W) + n * (size_t)K,
-                           static_cast<uint8_t*>(packed) + n * (size_t)(K / 2), static_cast<uint16_t*>(scales) + n * G,
-                           ngroups);
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
-    }
-    return 0;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    return few(N, K) ? launch_int4<64, 1>(W, packed, scales, N, K, st) : launch_int4<16, 2>(W, packed, scales, N, K, st);
 }
 
 int paia_quantize_int4_zp_g128(const void* W, void* packed, void* scales, void* zeros, int N, int K, void* stream)
@@ -329,22 +411,9 @@ int paia_quantize_int4_zp_g128(const void* W, void* packed, void* scales, void* 
     if (N <= 0 || K <= 0 || (K & 127) || !aligned(W, 16) || !aligned(packed, 16) || !aligned(scales, 2) ||
         zeros == nullptr)
         return -2;
-    const size_t G = (size_t)K / 128, ZB = (G + 1) / 2;
-    constexpr size_t kPerBlock = kQBlock / kWave * 2 * kQSteps;
-    const size_t step = slice_rows(ZB, kPerBlock);
-    for (size_t n = 0; n < (size_t)N; n += step) {
-        const size_t pairs = ((size_t)N - n < step ? (size_t)N - n : step) * ZB;
-        auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(blocks_for(pairs, kPerBlock)), dim3(kQBlock), 0, static_cast<hipStream_t>(stream),
-                               static_cast<const float*>(W) + n * (size_t)K,
-                               static_cast<uint8_t*>(packed) + n * (size_t)(K / 2), static_cast<uint16_t*>(scales) + n * G,
-                               static_cast<uint8_t*>(zeros) + n * ZB, (uint32_t)pairs, (int)G);
-        };
-        if (G & 1) launch(quantize_int4_zp_kernel<true>);
-        else launch(quantize_int4_zp_kernel<false>);
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
-    }
-    return 0;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    return few(N, K) ? launch_int4_zp<32, 1>(W, packed, scales, zeros, N, K, st)
+                     : launch_int4_zp<16, 2>(W, packed, scales, zeros, N, K, st);
 }
 
 }  // extern "C"

@@ -152,6 +152,58 @@ def test_quantize_int4_ragged_groups_and_scales_bitexact(oracle, gemv_lib, cuda,
     assert np.array_equal(s.cpu().view(torch.int16).numpy().view(np.uint16), s0)
 
 
+def int4_both(lib, oracle, W, cuda, what):
+    """Both INT4 formats of W (and of W with every other group 10^18 times larger for the asymmetric) against the oracle."""
+    N, K = W.shape
+    G = K // 128
+    for zp in (False, True):
+        A = W * np.where(np.arange(K) // 128 % 2, np.float32(1e18), np.float32(1)) if zp else W
+        d = _dev(A, cuda)
+        p = torch.empty(N, K // 2, dtype=torch.uint8, device=cuda)
+        s = torch.empty(N, G, dtype=torch.bfloat16 if zp else torch.float16, device=cuda)
+        z = torch.empty(N, (G + 1) // 2, dtype=torch.uint8, device=cuda)
+        note(f"quantize int4 {what} {N}x{K} zp={zp}")
+        if zp:
+            lib.quantize_int4_zp_g128(d.data_ptr(), p.data_ptr(), s.data_ptr(), z.data_ptr(), N, K)
+        else:
+            lib.quantize_int4_g128(d.data_ptr(), p.data_ptr(), s.data_ptr(), N, K)
+        torch.cuda.synchronize()
+        p0, s0, *z0 = oracle.quantize_int4_zp_g128(A) if zp else oracle.quantize_int4_g128(A)
+        assert np.array_equal(s.cpu().view(torch.int16).numpy().view(np.uint16), s0) and np.array_equal(p.cpu().numpy(), p0)
+        assert not zp or np.array_equal(z.cpu().numpy(), z0[0])
+
+
+# at most 2^20 weights, then more: groups alone, odd and even G, a wave or block part full
+@pytest.mark.parametrize("N,K", [(8192, 128), (8193, 128), (910, 1152), (911, 1152), (1366, 768), (263, 4096), (1, 1048704)])
+def test_quantize_int4_few_and_many_bitexact(oracle, gemv_lib, cuda, N, K):
+    rng = np.random.default_rng(N + K)
+    W = rng.standard_normal((N, K // 128, 128)) * rng.choice([1e-30, 1e-9, 1e-3, 1.0, 1e4], (N, K // 128, 1))
+    W = W.astype(np.float32).reshape(N, K)
+    ties = (np.arange(128) % 15 - 7 + 0.5).astype(np.float32)
+    ties[0] = 7.0                                          # amax 7 -> scale exactly 1: every w/s is a .5 tie
+    W[N // 2, :128], W[N - 1, -128:] = ties, 0.0
+    W[0, 5] = -0.0
+    int4_both(gemv_lib, oracle, W, cuda, "few and many")
+
+
+@pytest.mark.parametrize("N,K", [(1024, 1024), (1025, 1024), (1057, 976), (65537, 16), (3, 1008)])
+def test_quantize_fp8_few_and_many_bitexact(oracle, gemv_lib, cuda, N, K):
+    """Rows of at most 1024 weights in calls of up to 2^20 weights (a block each) and more (a wave each): every rounding case
+    where the row holds them, scales on both sides of the exact-quotient range elsewhere."""
+    rng = np.random.default_rng(N + K)
+    W = rng.standard_normal((N, K)) * rng.choice([1, 2.0 ** -54, 2.0 ** -100, 2.0 ** 68, 2.0 ** 120, 1e-38, 0.02], (N, 1))
+    W = W.astype(np.float32)
+    W[0, :] = 0.0
+    W[N - 1, 5] = -0.0
+    if K == 1024:
+        probe = e4m3_probe_rows(oracle)
+        W[7:7 + len(probe)] = probe
+    note(f"quantize fp8 few and many {N}x{K}")
+    q, s = run_fp8(gemv_lib, W, cuda)
+    q0, s0 = oracle.quantize_fp8_rowwise(W)
+    assert np.array_equal(s.view(np.uint32), s0.view(np.uint32)) and np.array_equal(q, q0)
+
+
 def test_quant_api_on_device_matches_definition(cuda):
     """paia_gemv.quant on a GPU tensor (the HIP kernels through the torch ops) == the torch definition on the CPU."""
     from paia_gemv import quant
