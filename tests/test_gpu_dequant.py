@@ -60,9 +60,16 @@ def test_dequant_bitexact_seeded(oracle, gemv_lib, cuda, fmt):
 
 @pytest.mark.parametrize("fmt,N,K", [("fp8", 515, 16), ("fp8", 9, 1360), ("fp8", 3, 2048), ("fp8", 2, 2064),
                                      ("fp8", 5, 4112), ("int4", 65, 128), ("int4", 4, 2048), ("int4", 3, 4224),
-                                     ("int4zp", 33, 896), ("int4zp", 7, 1920), ("int4zp", 2, 8320)])
+                                     ("int4zp", 33, 896), ("int4zp", 7, 1920), ("int4zp", 2, 8320),
+                                     # one step a lane: rows per block up to K = 512; then more than its weights
+                                     ("fp8", 3, 512), ("fp8", 7, 528), ("fp8", 5, 1024), ("fp8", 3, 1040),
+                                     ("int4", 9, 512), ("int4", 5, 640), ("int4zp", 3, 1152), ("fp8", 256, 4096),
+                                     ("fp8", 65537, 16), ("fp8", 772, 1360), ("fp8", 513, 2048), ("fp8", 509, 2064),
+                                     ("fp8", 256, 4112), ("int4", 12289, 128), ("int4", 769, 2048), ("int4", 373, 4224),
+                                     ("int4zp", 1756, 896), ("int4zp", 820, 1920), ("int4zp", 190, 8320)])
 def test_dequant_block_edges_bitexact(oracle, gemv_lib, cuda, fmt, N, K):
-    """Rows per block (K <= 2048, the last block part full) and blocks per row (the last part full); nothing past the end."""
+    """Rows per block (K <= 2048, or 512 in calls of few weights; the last block part full) and blocks per row (the last part
+    full); nothing past the end."""
     ops, np_ops = make(fmt, N, K)
     dev = to_device(ops, cuda)
     out = torch.full((N * K + 4096,), -7.0, dtype=torch.float32, device=cuda)
