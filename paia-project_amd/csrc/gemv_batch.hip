@@ -10,8 +10,8 @@
 // Variant knobs: P tiles of 16 rows per wave, U k-blocks (128 columns) of loads in flight per wave, W waves per block,
 // S waves sharing a tile along K (split-K inside the block), X how x reaches the matrix cores (0 staged in LDS per
 // K-chunk of up to 64 KiB, 1 loaded with the weights, 2 staged as for 0 in chunks of up to 80 KiB, or the device's
-// per-block LDS if less). variant < 0 is the library's choice: the tile kernel (gemv_tile.h), which has no table entry, or
-// paia_gemv_batch_pick_variant's entry where that is ahead (rows_ahead) or the tile kernel does not take the call.
+// per-block LDS if less). variant < 0 is the library's choice: the tile kernel (gemv_tile.h), which has no table entry,
+// or paia_gemv_batch_pick_variant's entry where that is ahead (table_ahead) or the tile kernel does not take the call.
 //
 // P = 0 marks the row-streaming kernel instead (gemv_rows_kernel: the M = 1 GEMV's weight stream and decode with one
 // accumulator per activation row, for M = 2..6, BF16 and FP8 also 7, 8): then U is its 1-KiB chunks per item, W its waves per
@@ -256,45 +256,84 @@ int pick(int kind, int M, int N, int K)
     return find(t, P, U, W, S, X);
 }
 
-// Where the row-streaming kernel stays ahead of the tile kernel (both measured, us, rows / tile): the tile kernel reads
-// 16 rows per wave and adds 8 waves' partial sums, which few tiles or few activation rows do not repay.
-//   * at most 128 tiles, where a block per tile leaves half the CUs idle: FP8 1000x3584 M = 2 3.22 / 3.86, M = 4 3.76 /
-//     4.12; BF16 M = 4 4.30 / 5.25, M = 7 and 8 even; INT4 M = 2 3.48 / 4.2, M = 3 even;
-//   * up to 1024 tiles of ordinary K, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even), FP8 M = 2
-//     (6144x4096 6.51 / 7.10, 10112x4096 9.19 / 10.09; M = 3 7.54 / 7.23), INT4 M = 2 up to 256 tiles (4096x4096
-//     4.84 / 5.2, 1455x1920 3.31 / 3.64, 3000x1536 4.44 / 3.31; 6144x4096 even), and the same at any N for K up to 2560 (BF16
-//     33000x2048 M = 2 21.5 / 22.4); and BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 /
-//     29.4, M = 5 29.2 / 30.7). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
-//     kernel's;
-//   * rows that are no multiple of 128 bytes, whose lines the tile kernel reads past their ends or carries through LDS: BF16 to
-//     M = 4 (40000x1512 21.3 / 23.9, 20000x5000 32.5 / 34.3, 60000x760 18.2 / 20.5; M = 5 34.2 / 32.8; above 2048 tiles and at
-//     any K to M = 6: 40408x2592 M = 5 34.4 / 36.5, 69979x2864 M = 6 66.8 / 70.7, 37492x13336 M = 4 146 / 158),
-//     FP8 M = 2 (40000x1520 12.9 / 15.0, 40000x3008 21.1 / 22.1; M = 3 23.1 / 22.6), while K <= 8192; beyond, BF16 at one to two tiles per CU to M = 6 (5000x12008 23.2 / 26.7);
-//   * INT4 M = 2 with long rows on many tiles (30000x14336 43.0 / 49.9, 15000x11008 20.1 / 22.0; 10000x14336 even,
-//     4096x14336 10.6 / 9.1) or a great many of ordinary K (100000x4096 44.4 / 45.7, 70000x7168 53.3 / 55.2; 60000x1920 even).
-bool rows_ahead(int kind, int M, int N, int K)
+// Where the table's kernel stays ahead of the tile kernel, which reads 16 rows per wave and adds the partial sums of a
+// block's waves: few tiles or few activation rows do not repay that. Times in us on MI355X (256 CUs), table / tile; the
+// bounds are in tiles per CU. The table's entry here is a row-streaming one wherever its x copies fit the LDS, and the
+// tile kernel takes the call where they do not (kRows) -- but for the one case whose entry is a matrix-core kernel
+// (kTable).
+//   * At most half a tile per CU, where a block per tile leaves half the CUs idle: BF16 to M = 7 (M = 4 4.30 / 5.25),
+//     at M = 8 even with rows of whole 128-byte lines, but split lines (next but one) are ahead from 1 MiB of weights
+//     on to 80 tiles, long rows from half of that to 112 (1168x2728 5.0 / 5.5, 592x3592 5.3 / 6.9, 350x9712 9.9 / 14.3,
+//     1376x7816 9.6 / 11.6; 160x1864 4.2 / 3.5, 1456x2984 6.4 / 5.9); FP8 to M = 4 (1000x3584 M = 2 3.22 / 3.86, M = 4
+//     3.76 / 4.12); INT4 M = 2 (3.48 / 4.2, 629x18048 8.3 / 10.6; M = 3 even) above K = 1536.
+//   * Ordinary K, up to 4 tiles per CU, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even),
+//     FP8 M = 2 (6144x4096 6.51 / 7.10; M = 3 7.54 / 7.23), and the same at any N for K up to 2560 (BF16 33000x2048 M =
+//     2 21.5 / 22.4); BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 / 29.4, M = 5 29.2 /
+//     30.7). Short rows (20000x1024 FP8 M = 2 7.61 / 6.13) and long ones (4096x14336 12.2 / 11.9) are the tile
+//     kernel's.
+//   * Split lines (rows that are no multiple of 128 bytes), which the tile kernel reads past their ends or carries
+//     through LDS: BF16 to M = 4 (40000x1512 21.3 / 23.9, 20000x5000 32.5 / 34.3), above 8 tiles per CU to M = 6
+//     (69979x2864 M = 6 66.8 / 70.7), K = 1544..2560 from 4 tiles per CU to M = 5 and up to K = 2048 to M = 6
+//     (19230x1864 M = 5 15.5 / 17.9; 24710x1384 M = 6 even), M = 6 at one to two tiles per CU and K > 8192 (5000x12008
+//     23.2 / 26.7). FP8 M = 2 (40000x1520 12.9 / 15.0), M = 3 above 4 tiles per CU (K > 4096: above 16) where the row
+//     streaming's 2 KiB items are three quarters full (43820x3696 30.3 / 35.4, but 36392x2160 20.8 / 17.7).
+//   * Rows 16 or 32 KiB apart (within 128 bytes per 16 KiB), which 16 rows read side by side find on few memory
+//     channels: BF16 16 KiB above 3 tiles per CU (25600x8192 M = 8 77 / 91, 14106x8192 M = 5 48 / 59; up to 3 the
+//     8-wave launch is 5 to 15% ahead), longer ones and FP8 above one (BF16 6760x16384 M = 5 49 / 75, FP8 12264x16256 M
+//     = 3 38.5 / 49.3); to M = 4 only up to 4 tiles per CU, as the block per tile beyond is even.
+//   * INT4 M = 2: up to a tile per CU and ordinary K (1455x1920 3.31 / 3.64), long rows on many tiles (30000x14336 43.0
+//     / 49.9, K = 6272..8192 on 1025..4096 tiles 0.88 to 0.98 of the tile kernel's, up to 6144 0.97 to 1.2), a great
+//     many of ordinary K (100000x4096 44.4 / 45.7, 70000x7168 53.3 / 55.2).
+//   * FP8 split lines of at most 960 bytes at M = 5..8 above 18 tiles per CU: the matrix-core kernel (119226x528 M = 7
+//     18.4 / 22.8).
+enum Ahead { kTile, kRows, kTable };
+Ahead table_ahead(int kind, int M, int N, int K)
 {
-    const int ntiles = (N + kTileRows - 1) / kTileRows;
-    const bool mid = K >= 2048 && K <= 8192;
-    if (kind >= 2)
-        return M == 2 && ((ntiles <= 256 && K > 1536 && K <= 8192) || (ntiles > 768 && K > 8192) ||
-                          (ntiles > 4096 && K >= 4096));
-    if (ntiles <= 128) return M <= (kind == 0 ? 7 : 4);
-    if ((kind == 0 ? 2 * K : K) % 128 != 0) {
-        if (K <= 8192 && M <= (kind != 0 ? 2 : 4)) return true;
-        if (kind == 0 && ntiles > 2048 && M <= 6) return true;
-        if (kind == 0 && K > 8192 && M == 6) return ntiles > 256 && ntiles <= 512;
+    const int cus = device_facts().cus > 0 ? device_facts().cus : 256;
+    const int64_t nt = ((int64_t)N + kTileRows - 1) / kTileRows;
+    auto rows = [](bool ahead) { return ahead ? kRows : kTile; };
+    if (kind >= 2) {
+        if (M != 2) return kTile;
+        if (2 * nt <= cus) return rows(K > 1536);
+        return rows((nt <= cus && K > 1536 && K <= 8192) || (nt > (K > 8192 ? 3 : 4) * cus && K > 6144) ||
+                    (nt > 16 * cus && K >= 4096));
     }
-    if (kind == 0 && K > 8192) return ntiles > 256 && ntiles <= 512 && M <= 5;
-    return mid && (ntiles <= 1024 || K <= 2560) && M <= (kind == 0 ? 3 : 2);
+    const bool bf16 = kind == 0, mid = K >= 2048 && K <= 8192;
+    const int row_bytes = bf16 ? 2 * K : K;
+    const bool split = row_bytes % 128 != 0;
+    if (2 * nt <= cus) {
+        if (!bf16 || M < 8) return rows(M <= (bf16 ? 7 : 4));
+        if (!split || M > 8) return kTile;
+        if (K < 4096) return rows(K >= 1408 && nt * K >= 32768 && 16 * nt <= 5 * cus);
+        return rows((K > 8192 || nt * K >= 16384) && 16 * nt <= 7 * cus);
+    }
+    if (split) {
+        if (K <= 8192 && M <= (bf16 ? 4 : 2)) return kRows;
+        if (!bf16) {
+            if (M == 3)
+                return rows(nt > (K <= 4096 ? 4 : 16) * cus && K <= 8192 && 4 * K >= 3 * ((K + 2047) / 2048 * 2048));
+            return M >= 5 && M <= 8 && K <= 960 && nt > 18 * cus ? kTable : kTile;
+        }
+        if (M <= 6 && nt > 8 * cus) return kRows;
+        if (K > 1536 && K <= 2560 && nt > 4 * cus && M <= (K <= 2048 ? 6 : 5)) return kRows;
+        if (K > 8192 && M == 6) return rows(nt > cus && nt <= 2 * cus);
+    } else {
+        const int apart = (row_bytes + 8192) / 16384, off = row_bytes - 16384 * apart;   // nearest multiple of 16 KiB
+        if (apart > 0 && off <= 128 * apart && -off <= 128 * apart && nt > (bf16 && apart == 1 ? 3 : 1) * cus &&
+            (M > 4 || nt <= 4 * cus))
+            return kRows;
+    }
+    if (bf16 && K > 8192) return rows(nt > cus && nt <= 2 * cus && M <= 5);
+    return rows(mid && (nt <= 4 * cus || K <= 2560) && M <= (bf16 ? 3 : 2));
 }
 
 int batch_impl(int kind, BatchParams p, int variant, void* stream)
 {
     const Table t = table(kind);
     if (variant < 0) {   // the library's choice: the tile kernel, or the table's best where that is ahead or it refuses
-        if (rows_ahead(kind, p.M, p.N, p.K)) variant = pick(kind, p.M, p.N, p.K);
-        if (variant < 0 || t.v[variant].P != 0) {
+        const Ahead ahead = p.M > 1 ? table_ahead(kind, p.M, p.N, p.K) : kTable;
+        if (ahead != kTile) variant = pick(kind, p.M, p.N, p.K);
+        if (variant < 0 || (ahead == kRows && t.v[variant].P != 0)) {
             const int rc = launch_tile_picked(kind, p, static_cast<hipStream_t>(stream));
             if (rc != kTileRefused) return rc;
             variant = pick(kind, p.M, p.N, p.K);

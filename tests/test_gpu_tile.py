@@ -189,3 +189,43 @@ def test_row_forms(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
     keep = torch.ones(N, dtype=torch.bool, device=cuda)
     keep[bad] = False
     assert torch.equal(y3[:, keep].view(torch.int16), y[:, keep].view(torch.int16))
+
+
+# Both sides of the rule that keeps a call on the variant table's kernel: (format, M, N, K, on the table's kernel). On the
+# tile kernel's side only calls of 10^5 outputs, enough for some to differ.
+ROUTES = [("bf16", 8, 592, 3592, True), ("bf16", 8, 350, 9712, True), ("bf16", 8, 64, 6136, True),
+          ("bf16", 6, 18428, 1872, True), ("bf16", 5, 19230, 1864, True), ("bf16", 6, 19230, 2104, False),
+          ("bf16", 5, 14106, 8192, True), ("bf16", 4, 14106, 8256, True), ("bf16", 4, 17000, 8192, False),
+          ("bf16", 8, 10000, 8192, False), ("bf16", 8, 14106, 8320, False), ("fp8", 3, 43820, 3696, True),
+          ("fp8", 3, 36392, 2160, False), ("fp8", 3, 12264, 16256, True), ("fp8", 5, 12264, 16256, False),
+          ("fp8", 7, 74000, 528, True), ("fp8", 7, 73000, 528, False), ("fp8", 9, 74000, 528, False),
+          ("int4", 2, 629, 18048, True), ("int4zp", 2, 629, 18048, True), ("int4", 2, 17000, 7552, True),
+          ("int4zp", 2, 17000, 6016, False)]
+
+
+@pytest.mark.parametrize("fmt,M,N,K,table", ROUTES)
+def test_route(gemv_lib, cuda, fmt, M, N, K, table):
+    """Where the table's kernel is the faster one a default call gives its bits; elsewhere the tile kernel's sums, split
+    over a block's waves, round another way somewhere. Both are within twice the rounding of bf16."""
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the bounds are in tiles per CU: these sizes are for 256")
+    g = torch.Generator(device=cuda).manual_seed(N + K)
+    dev = {"N": N}
+    if fmt == "bf16":
+        dev["W"] = torch.randn(N, K, dtype=torch.bfloat16, device=cuda, generator=g)
+    elif fmt == "fp8":
+        dev["Wq"] = torch.randint(0, 0x78, (N, K), dtype=torch.uint8, device=cuda, generator=g)
+        dev["scale"] = torch.rand(N, device=cuda, generator=g)
+    else:
+        dev["Wq"] = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device=cuda, generator=g)
+        dev["scales"] = torch.rand(N, K // 128, device=cuda, generator=g).to(
+            torch.float16 if fmt == "int4" else torch.bfloat16)
+        dev["zeros"] = torch.randint(0, 256, (N, (K // 128 + 1) // 2), dtype=torch.uint8, device=cuda, generator=g)
+    x = x_rows(M, K, 11).to(cuda)
+    note(f"route {fmt} M={M} {N}x{K}")
+    y = run_batch(gemv_lib, fmt, dev, x)
+    want = run_batch(gemv_lib, fmt, dev, x, gemv_lib.batch_pick_variant(fmt, M, N, K))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16)) == table
+    d = (y.float() - want.float()).norm() / want.float().norm()
+    assert d < 2.0 ** -8
