@@ -10,7 +10,8 @@ the reference. Extra, beyond the reference's test:
   * BF16 and FP8 with all-zero weights must give exactly +0 in every row (every product is 0);
   * the INT4 kernels compute s * (sum (128+q) x - (128+z) sum x), a cancellation of two terms of size ~128 |sum x|:
     zero weights with |x| ~ 100 (x ~ 100 N(0,1)) must stay within the gate;
-  * the naive and unfused INT4 controls and the small-batch pick (M = 2, 4, 16) see the same operands;
+  * the naive and unfused INT4 controls and the small-batch calls (M = 2, 4, 8, 16; the library's choice and the
+    table's pick) see the same operands;
   * activations over a wide range of magnitudes, random signs: "wide" (|x| = 2^-50 .. 2^50), "bigx" (2^50 .. 2^63),
     "low" (2^-40 .. 2^-20), "tiny" (every |x| in 2^-120 .. 2^-55) and "huge" (2^60 .. 2^99, outputs still finite in
     bf16). The INT4 kernels that stage x read the nibbles as bf16 subnormals against x scaled by a power of two: 2^64
@@ -162,33 +163,39 @@ def test_int4_controls_on_special_operands(oracle, gemv_lib, cuda, special):
 @pytest.mark.parametrize("special", ["zeros", "large"])
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_batch_pick_on_special_operands(oracle, gemv_lib, cuda, fmt, special):
-    """The small-batch entry points at the library's pick, M = 2, 4, 16, every activation row the special x times a
-    per-row factor (so rows differ), each row gated against the oracle."""
+    """The small-batch entry points at the library's choice (the tile kernel; at few activation rows the row-streaming one)
+    and at the variant table's pick, M = 2, 4, 8, 16, every activation row the special x times a per-row factor (so rows
+    differ), each row gated against the oracle. BF16 and FP8 zero weights give zero in every row."""
     o, np_ops, dev = prepared(oracle, fmt, special, cuda)
     L = gemv_lib
-    for M in (2, 4, 16):
+    for M in (2, 4, 8, 16):
         f = torch.linspace(1.0, -1.0, M)
         xs = (o["x"].float()[None, :] * f[:, None]).to(torch.bfloat16)
         xd = xs.to(cuda)
-        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
-        v = L.batch_pick_variant(fmt, M, N, K)
-        note(f"special batch {special} {fmt} M={M} variant={v}")
-        if fmt == "bf16":
-            L.batch_bf16(dev["W"].data_ptr(), xd.data_ptr(), None, y.data_ptr(), M, N, K, v)
-        elif fmt == "fp8":
-            L.batch_fp8(dev["Wq"].data_ptr(), dev["scale"].data_ptr(), xd.data_ptr(), None, y.data_ptr(), M, N, K, v)
-        elif fmt == "int4":
-            L.batch_int4(dev["Wq"].data_ptr(), dev["scales"].data_ptr(), xd.data_ptr(), y.data_ptr(), M, N, K, v)
-        else:
-            L.batch_int4_zp(dev["Wq"].data_ptr(), dev["scales"].data_ptr(), dev["zeros"].data_ptr(), xd.data_ptr(),
-                            None, y.data_ptr(), M, N, K, v)
-        torch.cuda.synchronize()
-        yb = bits16(y).reshape(M, N)
         xb = xs.view(torch.int16).numpy().view(np.uint16)
+        refs = []
         for m in range(M):
             row_ops = dict(np_ops, x=np.ascontiguousarray(xb[m]))
             row_ops["_ref"] = oracle_ref(oracle, fmt, row_ops)
-            gate(oracle, fmt, row_ops, yb[m].copy(), f"batch {special} {fmt} M={M} row {m}")
+            refs.append(row_ops)
+        for v in (-1, L.batch_pick_variant(fmt, M, N, K)):
+            y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+            note(f"special batch {special} {fmt} M={M} variant={v}")
+            if fmt == "bf16":
+                L.batch_bf16(dev["W"].data_ptr(), xd.data_ptr(), None, y.data_ptr(), M, N, K, v)
+            elif fmt == "fp8":
+                L.batch_fp8(dev["Wq"].data_ptr(), dev["scale"].data_ptr(), xd.data_ptr(), None, y.data_ptr(), M, N, K, v)
+            elif fmt == "int4":
+                L.batch_int4(dev["Wq"].data_ptr(), dev["scales"].data_ptr(), xd.data_ptr(), y.data_ptr(), M, N, K, v)
+            else:
+                L.batch_int4_zp(dev["Wq"].data_ptr(), dev["scales"].data_ptr(), dev["zeros"].data_ptr(), xd.data_ptr(),
+                                None, y.data_ptr(), M, N, K, v)
+            torch.cuda.synchronize()
+            yb = bits16(y).reshape(M, N)
+            for m in range(M):
+                gate(oracle, fmt, refs[m], yb[m].copy(), f"batch {special} {fmt} M={M} v{v} row {m}")
+            if special == "zeros" and fmt in ("bf16", "fp8"):
+                assert not y.any()
 
 
 @pytest.mark.parametrize("special", ["tiny", "huge", "wide", "low"])

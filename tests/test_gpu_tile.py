@@ -85,6 +85,43 @@ def test_replays_and_rows(gemv_lib, cuda, fmt):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "int4", "int4zp"])
+@pytest.mark.parametrize("M", [9, 16])
+def test_rows_of_infinities_and_nan(gemv_lib, cuda, fmt, M):
+    """Activation rows that hold infinities and NaN beside finite ones: not finite themselves, and every other row keeps its
+    bits."""
+    N, K = 2070, 1152
+    ops, _ = make(fmt, N, K, bias=fmt != "int4")
+    dev = to_device(ops, cuda)
+    x = x_rows(M, K, 41).to(cuda)
+    note(f"tile rows of infinities {fmt} M={M}")
+    want = run_batch(gemv_lib, fmt, dev, x)
+    bad = x.clone()
+    bad[1, 5], bad[4, K - 1], bad[M - 1, 700] = float("inf"), float("nan"), float("-inf")
+    y = run_batch(gemv_lib, fmt, dev, bad)
+    torch.cuda.synchronize()
+    keep = [m for m in range(M) if m not in (1, 4, M - 1)]
+    assert torch.equal(y[keep].view(torch.int16), want[keep].view(torch.int16))
+    # a weight of zero times an infinity is a NaN: no output of these rows is finite
+    assert not torch.isfinite(y[[1, 4, M - 1]]).any()
+
+
+@pytest.mark.parametrize("fmt", ["int4", "int4zp"])
+@pytest.mark.parametrize("N,K,M", [(33, 262144, 16), (16, 300032, 3)])
+def test_metadata_beyond_the_lds(oracle, gemv_lib, cuda, fmt, N, K, M):
+    """Rows whose scales and zero points do not fit the block's LDS even for one tile (above K = 230912 at M = 16, 277504 at
+    M <= 4): the call goes to the variant table's kernel."""
+    ops, np_ops = make(fmt, N, K)
+    x = x_rows(M, K, 43)
+    note(f"tile metadata beyond LDS {fmt} M={M} {N}x{K}")
+    dev = to_device(ops, cuda)
+    y = run_batch(gemv_lib, fmt, dev, x.to(cuda))
+    want = run_batch(gemv_lib, fmt, dev, x.to(cuda), gemv_lib.batch_pick_variant(fmt, M, N, K))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    check_rows(oracle, y, oracle_rows(oracle, fmt, np_ops, xbits(x)), f"{fmt} M={M} {N}x{K}")
+
+
 @pytest.mark.parametrize("fmt", ["int4", "int4zp"])
 @pytest.mark.parametrize("lo,hi", [(-125, -112), (-120, -55), (-50, 50), (60, 99), (100, 120)])
 def test_int4_extreme_x(oracle, gemv_lib, cuda, fmt, lo, hi):
@@ -159,6 +196,18 @@ def test_int4zp_largest_scales(oracle, gemv_lib, cuda):
                                            (4112, 2048 + 64, 9), (13000, 1408 + 80, 16), (8200, 2176 - 32, 8),
                                            (4112, 1024 + 112, 16), (528, 1024 + 80, 12), (1041, 2400 + 16, 9), (8200, 16, 9), (4112, 9200, 8)])
 def test_row_forms(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
+    row_form(oracle, gemv_lib, cuda, fmt, N, row_bytes, M)
+
+
+# The same with four activation rows staged: line by line with three and seven tiles per wave, as a block per tile, and
+# in 8-wave blocks
+@pytest.mark.parametrize("fmt,N,row_bytes,M", [("fp8", 12000, 3600, 3), ("fp8", 12001, 3600, 4), ("fp8", 25000, 2000, 4),
+                                               ("fp8", 17000, 5008, 4), ("bf16", 9001, 16400, 4)])
+def test_row_forms_few_rows(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
+    row_form(oracle, gemv_lib, cuda, fmt, N, row_bytes, M)
+
+
+def row_form(oracle, gemv_lib, cuda, fmt, N, row_bytes, M):
     """Also from weights 16 bytes past a line (bit for bit the same), and with a row of NaN between finite ones: rows that share
     its lines keep their results."""
     K = row_bytes // (2 if fmt == "bf16" else 1)
@@ -200,7 +249,9 @@ ROUTES = [("bf16", 8, 592, 3592, True), ("bf16", 8, 350, 9712, True), ("bf16", 8
           ("fp8", 3, 36392, 2160, False), ("fp8", 3, 12264, 16256, True), ("fp8", 5, 12264, 16256, False),
           ("fp8", 7, 74000, 528, True), ("fp8", 7, 73000, 528, False), ("fp8", 9, 74000, 528, False),
           ("int4", 2, 629, 18048, True), ("int4zp", 2, 629, 18048, True), ("int4", 2, 17000, 7552, True),
-          ("int4zp", 2, 17000, 6016, False)]
+          ("int4zp", 2, 17000, 6016, False),
+          # six tiles per wave: metadata beyond the LDS above K = 37376
+          ("int4", 16, 24576, 38400, True), ("int4zp", 16, 24576, 37376, False)]
 
 
 @pytest.mark.parametrize("fmt,M,N,K,table", ROUTES)
