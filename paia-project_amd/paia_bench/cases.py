@@ -54,8 +54,9 @@ def kind_of(fmt: str) -> str:
 
 
 class GemvCase:
-    """mode: 'fused' (the M = 1 kernels), 'naive' / 'unfused' (INT4 controls), or 'batch' (the small-batch matrix-core
-    kernels, M = 1..16 activation rows; `variant` then indexes lib.variants_batch[fmt])."""
+    """mode: 'fused' (the M = 1 kernels), 'naive' / 'unfused' (INT4 controls), or 'batch' (the small-batch entry points,
+    M = 1..16 activation rows; `variant` then indexes lib.variants_batch[fmt], or is -1 for what a call that leaves it to
+    the library runs: the default, as the tile kernel has no index)."""
 
     def __init__(self, lib, fmt: str, N: int, K: int, bias: bool = False, variant: int | None = None,
                  mode: str = "fused", name: str | None = None, M: int = 1):
@@ -65,7 +66,7 @@ class GemvCase:
         if variant is not None:
             self.variant = int(variant)
         elif mode == "batch":
-            self.variant = lib.batch_pick_variant(fmt, M, N, K)
+            self.variant = -1
         else:
             self.variant = lib.pick_variant(fmt, N, K)
         self.copies: list = []

@@ -87,7 +87,8 @@ def main(argv=None):
     ap.add_argument("--out", default=None)
     ap.add_argument("--write-tuned", default=None)
     ap.add_argument("--batch", default="", help="M values: time the small-batch kernels (variants P,U,W,S,X)")
-    ap.add_argument("--pick-only", action="store_true", help="time only the library's choice for each cell")
+    ap.add_argument("--pick-only", action="store_true",
+                    help="time only the library's choice for each cell (small batch: the call with variant -1)")
     ap.add_argument("--merge", nargs="+", default=None,
                     help="no timing: merge these --out files (fastest per cell) into --write-tuned")
     a = ap.parse_args(argv)
@@ -102,9 +103,11 @@ def main(argv=None):
         write_tuned(Path(a.write_tuned), a.fmt, merged)
         return 0
 
+    batch = [int(m) for m in a.batch.split(",") if m]
+    if batch and a.pick_only and a.write_tuned:
+        raise SystemExit("--write-tuned takes variants; a default small-batch call need not run one")
     lib = load_lib()
     dev = torch.device("cuda:0")
-    batch = [int(m) for m in a.batch.split(",") if m]
     if batch:
         fam = lib.variants_batch[a.fmt]
         knobs = "PUWSX"
@@ -144,10 +147,9 @@ def main(argv=None):
         print(f"[sweep] {a.fmt} {tag}{nm} {N}x{K}: {rot['n_copies']} copies, built in {time.time() - t0:.1f}s",
               flush=True)
         rows_res = []
-        for v in fam:
-            if not keep(v):
-                continue
-            if a.pick_only and v["id"] != case.variant:
+        default = a.pick_only and batch
+        for v in [{"id": -1}] if default else fam:
+            if not default and (not keep(v) or a.pick_only and v["id"] != case.variant):
                 continue
             case.variant = v["id"]
             try:
@@ -161,9 +163,9 @@ def main(argv=None):
             t = time_per_call_us(case.call, rot["n_copies"], target_ms=a.target_ms, samples=a.samples,
                                  warmup_ms=20.0)
             gbps = case.bytes()["total"] / (t["us"] * 1e-6) / 1e9
-            rows_res.append({"variant": {k: v[k] for k in knobs}, "id": v["id"], "us": t["us"], "gbps": gbps,
+            rows_res.append({"variant": {k: v[k] for k in knobs if k in v}, "id": v["id"], "us": t["us"], "gbps": gbps,
                              "cv": t.get("us_cv")})
-            print("  " + " ".join(f"{k}={v[k]}" for k in knobs) + f": {t['us']:8.2f} us {gbps:7.0f} GB/s "
+            print("  " + (" ".join(f"{k}={v[k]}" for k in knobs if k in v) or "default") + f": {t['us']:8.2f} us {gbps:7.0f} GB/s "
                   f"({100 * gbps / HBM_PEAK_GBPS:4.1f}%)", flush=True)
         rows_res.sort(key=lambda r: r["us"])
         key = f"{M}x{N}x{K}" if batch else f"{N}x{K}"

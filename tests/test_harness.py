@@ -309,3 +309,17 @@ def test_pmc_summary_of_every_case_assigns_dispatches_in_order(tmp_path):
     (tmp_path / "plan.json").write_text(json.dumps(plan))
     with pytest.raises(SystemExit):
         pmc.main(args)
+
+
+def test_small_batch_cases_time_the_default_call():
+    """A small-batch case without a variant makes the call that leaves it to the library (variant -1); the entry
+    lib.batch_pick_variant names is not what such a call need run."""
+    c = GemvCase(_NoLib(), "fp8", 4096, 4096, mode="batch", M=16)
+    assert c.variant == -1
+    assert GemvCase(_NoLib(), "fp8", 4096, 4096, mode="batch", M=16, variant=3).variant == 3
+
+
+def test_sweep_keeps_default_calls_out_of_the_tuned_table(tmp_path):
+    from paia_bench import sweep
+    with pytest.raises(SystemExit, match="default"):
+        sweep.main(["--fmt", "fp8", "--batch", "4", "--pick-only", "--write-tuned", str(tmp_path / "t.json")])
