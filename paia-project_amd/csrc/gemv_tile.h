@@ -15,8 +15,8 @@
 //     against bank conflicts) to bring it into the MFMA layout: no block barrier, and LDS operations of a wave complete in
 //     order, so a slot can be rewritten behind the reads of its last contents. Weights are then worth the streaming (nt)
 //     policy: 25.1 -> 21.9 us on that shape, where it cost gemv_batch_kernel 10%.
-//   * K is split over the W waves of the block. A wave takes its stages (BF16 64 columns, the others 128) for P tiles at a
-//     time, so each x fragment it brings in is used P times, with D stages of loads in flight; the W partial tiles are
+//   * K is split over S waves of the block. A wave takes its stages (BF16 64 columns, the others 128) for P tiles at a
+//     time, so each x fragment it brings in is used P times, with D stages of loads in flight; the S partial tiles are
 //     added in a fixed order after the one block barrier at the end. The operands of that epilogue (row scale, bias) are
 //     loaded before the first weight load: loaded at the end they cost 1.2 us per launch (FP8 4096x4096 M = 4 6.98 -> 5.68).
 //   * INT4 scales and zero points: per-group loads in the loop would touch 16 rows each, as many lines as the weights
@@ -51,7 +51,7 @@ struct TileParams {
     int M, N, K;
     uint32_t row_bytes, meta_bytes, zbytes;
     int stages;             // ceil(K / columns per stage)
-    int tq, tr;             // block b takes tiles tq*b + min(b, tr) .. of the next block: tq or tq + 1
+    int tq, tr;             // unit u (a group of S waves) takes tiles tq*u + min(u, tr) .. of its next unit: tq or tq + 1
     int chunks;             // INT4: ceil(G / 4), four-group chunks per row
     uint32_t chunk_mul;     // ceil(2^32 / chunks): i / chunks as the high word of i * chunk_mul (i * chunks < 2^32)
     int mstride;            // INT4: words per group in LDS (the most rows a block takes, plus one against bank conflicts)
@@ -114,13 +114,13 @@ __device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w, float scale)
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, HI));
 }
 
-// P tiles per block, W waves sharing them along K, D stages in flight per wave, MT activation rows staged (4, 8 or 16 >=
-// M), AUX cache policy of the weight loads, IL: the waves take the stages in turn
+// P tiles per unit, S waves sharing them along K (W / S units per block), D stages in flight per wave, MT activation
+// rows staged (4, 8 or 16 >= M), AUX cache policy of the weight loads, IL: a unit's waves take the stages in turn
 // (neighbouring waves read neighbouring bytes of a row) rather than a contiguous range each.
 // RING (BF16, FP8; not IL): for rows that are no multiple of 128 bytes, where a stage's 128 bytes of a row lie in two lines
 // and each line would be read twice (and fetched 1.6 times: with nt it is gone by the second read). A wave reads the lines of
 // its range once each, whole, and a stage takes its columns from the row's last two lines in LDS.
-template <int F, int P, int W, int D, int MT, int AUX, bool IL, bool RING>
+template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL, bool RING>
 __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams p)
 {
     using T = TileFmt<F>;
@@ -129,16 +129,18 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     constexpr int XL = (MT + XR - 1) / XR;            // x loads per stage
     constexpr int WP = RB / 16, WR = kWave / WP;      // 16-byte pieces per weight row and stage, rows per load
     constexpr int XP = 2 * C / 16;                    // 16-byte pieces per x row and stage
+    constexpr int kUnits = W / S;
     constexpr int kSlots = RING || P < kTileSlots ? P : kTileSlots;
     constexpr uint32_t kXBytes = (uint32_t)MT * 2u * C, kSlotBytes = (uint32_t)kTileRows * RB * (RING ? 2u : 1u);
     constexpr uint32_t kWaveBytes = tile_wave_bytes<F, P, MT, RING>();
-    constexpr int kOuts = (P + W - 1) / W;            // tiles a wave reduces and stores
-    static_assert(MT == 4 || MT == 8 || MT == 16, "launch shape");
+    constexpr int kOuts = (kUnits * P + W - 1) / W;   // tiles a wave reduces and stores
+    static_assert(W % S == 0 && (MT == 4 || MT == 8 || MT == 16), "launch shape");
     static_assert(!RING || (!I4 && !IL), "lines of contiguous ranges");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
     const int lane = lane_id(), wave = wave_id();
     const int ln = lane & 15, lh = lane >> 4;
+    const int split = wave % S, unit = wave / S;
     // logical block: each of the 8 XCDs (workgroups are dealt to them in turn) takes a contiguous range of tiles, so the
     // lines of y, scales and bias that tiles share are touched by one L2
     int lb = (int)blockIdx.x;
@@ -146,17 +148,18 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
         const int g = (int)gridDim.x, xcd = lb % 8, per = g / 8, rem = g % 8;
         lb = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + lb / 8;
     }
-    auto tile_at = [&](int b) { return b * p.tq + min(b, p.tr); };
-    const int t0 = tile_at(lb), nt = tile_at(lb + 1) - t0;   // this block's tiles, nt <= P
-    const int k0 = IL ? wave : wave * p.stages / W;
-    const int n = IL ? (p.stages - wave + W - 1) / W : (wave + 1) * p.stages / W - k0;   // this wave's stages
+    auto tile_at = [&](int u) { return u * p.tq + min(u, p.tr); };
+    const int u0 = lb * kUnits;
+    const int t0 = tile_at(u0 + unit), nt = tile_at(u0 + unit + 1) - t0;   // this unit's tiles, nt <= P
+    const int k0 = IL ? split : split * p.stages / S;
+    const int n = IL ? (p.stages - split + S - 1) / S : (split + 1) * p.stages / S - k0;   // this wave's stages
     // RING: line t = 0 only fills the ring, line t > 0 completes stage t - 1 of the range
     const int nl = RING ? (n > 0 ? n + 1 : 0) : n;
-    auto stage_at = [&](int t) { return IL ? k0 + t * W : (RING ? k0 + t - 1 : k0 + t); };
+    auto stage_at = [&](int t) { return IL ? k0 + t * S : (RING ? k0 + t - 1 : k0 + t); };
 
     // INT4 metadata of the block's rows: item i is four groups of one row
-    const int brows = I4 ? max(0, min(nt * kTileRows, p.N - t0 * kTileRows)) : 0;
-    const size_t brow0 = brows > 0 ? (size_t)(t0 * kTileRows) : 0;
+    const int bt0 = tile_at(u0), brows = I4 ? max(0, min((tile_at(u0 + kUnits) - bt0) * kTileRows, p.N - bt0 * kTileRows)) : 0;
+    const size_t brow0 = brows > 0 ? (size_t)(bt0 * kTileRows) : 0;
     const __amdgpu_buffer_rsrc_t rsm = make_rsrc(p.meta + (I4 ? brow0 * p.meta_bytes : 0),
                                                  I4 ? (uint32_t)brows * p.meta_bytes : 0u);
     const __amdgpu_buffer_rsrc_t rsz = make_rsrc(F == kI4ZP ? p.zeros + brow0 * p.zbytes : p.W,
@@ -207,13 +210,14 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     Meta m0;
     if constexpr (I4) m0 = meta_load((int)threadIdx.x);
 
-    // Epilogue operands of the tiles this wave stores: tile number q = wave, wave + W, ...
+    // Epilogue operands of the tiles this wave stores: (unit, tile) number q = wave, wave + W, ...
     uint32_t ep_scale[kOuts], ep_bias[kOuts];
     int ep_row[kOuts];
 #pragma unroll
     for (int e = 0; e < kOuts; ++e) {
-        const int q = wave + e * W;
-        const int row = q < nt ? (t0 + q) * kTileRows + ln : p.N;
+        const int q = wave + e * W, qu = q / P, qt = q - qu * P;
+        const int a0 = tile_at(u0 + qu), a1 = tile_at(u0 + qu + 1);
+        const int row = q < kUnits * P && a0 + qt < a1 ? (a0 + qt) * kTileRows + ln : p.N;
         const uint32_t off = row < p.N ? (uint32_t)row : (kOOB >> 2);
         ep_row[e] = row;
         ep_scale[e] = 0u;
@@ -308,9 +312,9 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                        0, 0);
     };
-    // INT4: this lane's metadata words. Rows past N and tiles past the block's read words that nothing wrote; their sums are
+    // INT4: this lane's metadata words. Rows past N and tiles past the unit's read words that nothing wrote; their sums are
     // meaningless, stay in their own D columns and are not stored.
-    const uint32_t* mw = md + (I4 ? ln : 0);
+    const uint32_t* mw = md + (I4 ? (t0 - bt0) * kTileRows + ln : 0);
 
     f32x4 acc[P];
 #pragma unroll
@@ -403,18 +407,18 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
     for (int d = 0; d < D; ++d)
         if (t + d < nl) consume(buf[(d + kFirst) % D], t + d);
 
-    // Partial tiles to the wave's own region, one barrier, then tile q is added up in split order and stored.
+    // Partial tiles to the wave's own region, one barrier, then (unit, tile) q is added up in split order and stored.
 #pragma unroll
     for (int t2 = 0; t2 < P; ++t2) *reinterpret_cast<f32x4*>(lds + t2 * 1024 + lane * 16) = acc[t2];
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < kOuts; ++e) {
-        const int q = wave + e * W;
-        if (q >= P || ep_row[e] >= p.N) continue;
-        const unsigned char* part = smem + p.wave_off + q * 1024 + lane * 16;
+        const int q = wave + e * W, qu = q / P, qt = q - qu * P;
+        if (q >= kUnits * P || ep_row[e] >= p.N) continue;
+        const unsigned char* part = smem + p.wave_off + (uint32_t)(qu * S) * kWaveBytes + qt * 1024 + lane * 16;
         f32x4 v = *reinterpret_cast<const f32x4*>(part);
 #pragma unroll
-        for (int s = 1; s < W; ++s) v += *reinterpret_cast<const f32x4*>(part + (uint32_t)s * kWaveBytes);
+        for (int s = 1; s < S; ++s) v += *reinterpret_cast<const f32x4*>(part + (uint32_t)s * kWaveBytes);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int m = 4 * lh + c;
@@ -435,11 +439,12 @@ __global__ void __launch_bounds__(W * kWave, W / 4) gemv_tile_kernel(TileParams 
 // A call the tile kernel does not take (shape, alignment, LDS, or a rule of the choice): nothing was launched.
 constexpr int kTileRefused = -100;
 
-// The launch on `st` with `blocks` blocks (raised to one per P tiles). Returns 0, kTileRefused when the block's
+// The launch on `st` with `blocks` blocks (raised to one per kUnits * P tiles). Returns 0, kTileRefused when the block's
 // metadata does not fit the LDS, or a hipError_t.
-template <int F, int P, int W, int D, int MT, int AUX, bool IL, bool RING>
+template <int F, int P, int W, int S, int D, int MT, int AUX, bool IL, bool RING>
 int launch_tile(const BatchParams& b, int blocks, hipStream_t st)
 {
+    constexpr int kUnits = W / S;
     TileParams p{};
     p.W = b.W;
     p.meta = static_cast<const uint8_t*>(b.meta);
@@ -455,16 +460,17 @@ int launch_tile(const BatchParams& b, int blocks, hipStream_t st)
     p.zbytes = b.zbytes;
     p.stages = (b.K + TileFmt<F>::kCols - 1) / TileFmt<F>::kCols;
     const int ntiles = (b.N + kTileRows - 1) / kTileRows;
-    const int fewest = (ntiles + P - 1) / P;
+    const int fewest = (ntiles + kUnits * P - 1) / (kUnits * P);
     if (blocks < fewest) blocks = fewest;
-    p.tq = ntiles / blocks;
-    p.tr = ntiles % blocks;
+    p.tq = ntiles / (blocks * kUnits);
+    p.tr = ntiles % (blocks * kUnits);
     uint64_t lds = 0;
     if (TileFmt<F>::kI4F) {
         const int G = b.K / kBlockCols;
         p.chunks = G > 8 ? (G + 3) / 4 : 2;   // at least two: chunk_mul is 32 bits
         p.chunk_mul = (uint32_t)(((1ull << 32) + p.chunks - 1) / p.chunks);
-        p.mstride = kTileRows * P + 1;
+        // the last unit's first tile, and the P tiles a wave's reads span from there
+        p.mstride = kTileRows * ((kUnits - 1) * (p.tq + (p.tr ? 1 : 0)) + P) + 1;
         p.wide = G % 4 == 0 && aligned(b.meta, 8) && (F != kI4ZP || aligned(b.zeros, 2));
         lds = ((uint64_t)p.chunks * 4u * (uint64_t)p.mstride * 4u + 127u) & ~127ull;
         if (lds > rows_max_lds()) return kTileRefused;
@@ -472,7 +478,7 @@ int launch_tile(const BatchParams& b, int blocks, hipStream_t st)
     p.wave_off = (uint32_t)lds;
     lds += (uint64_t)W * tile_wave_bytes<F, P, MT, RING>();
     if (lds > rows_max_lds()) return kTileRefused;
-    auto kernel = &gemv_tile_kernel<F, P, W, D, MT, AUX, IL, RING>;
+    auto kernel = &gemv_tile_kernel<F, P, W, S, D, MT, AUX, IL, RING>;
     if (lds > kMaxLds) {   // beyond the default dynamic-LDS limit: raise it once per device for this kernel
         static std::atomic<uint64_t> raised{0};
         int dev = 0;

@@ -48,12 +48,12 @@ template <int F, int MT, int P, int W, int D>
 int launch_d(const BatchParams& b, int blocks, hipStream_t st)
 {
     if constexpr (TileFmt<F>::kI4F) {
-        return launch_tile<F, P, W, D, MT, 0, true, false>(b, blocks, st);
+        return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);
     } else {
         switch (row_form<F, P>(b)) {
-        case kLines: return launch_tile<F, P, W, D, MT, 2, P == 1, false>(b, blocks, st);
-        case kRing: return launch_tile<F, P, W, D, MT, 2, false, true>(b, blocks, st);
-        default: return launch_tile<F, P, W, D, MT, 0, true, false>(b, blocks, st);
+        case kLines: return launch_tile<F, P, W, W, D, MT, 2, P == 1, false>(b, blocks, st);
+        case kRing: return launch_tile<F, P, W, W, D, MT, 2, false, true>(b, blocks, st);
+        default: return launch_tile<F, P, W, W, D, MT, 0, true, false>(b, blocks, st);
         }
     }
 }

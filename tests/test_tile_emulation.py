@@ -1,4 +1,4 @@
-"""The tile kernel's index arithmetic (paia-project_amd/csrc/gemv_tile.h) replayed on the CPU: every tile has one block and
+"""The tile kernel's index arithmetic (paia-project_amd/csrc/gemv_tile.h) replayed on the CPU: every tile has one unit and
 every stage one wave, the XCD order is a permutation, the metadata items divide exactly and stay in their LDS words, and the
 swizzled LDS layouts bring each lane the columns its MFMA step takes, without a bank conflict among 8 rows. Also its INT4
 decode: nibbles as e4m3 bytes, their pairs against the re-paired activations, and the powers of two on the way."""
@@ -11,12 +11,13 @@ import pytest
 from test_batch_emulation import step_col
 
 
-@pytest.mark.parametrize("tiles,blocks", [(1, 1), (257, 129), (632, 211), (2063, 768), (1792, 448), (7, 2), (6250, 1563)])
-def test_tiles_and_blocks(tiles, blocks):
-    tq, tr = divmod(tiles, blocks)
-    at = lambda b: b * tq + min(b, tr)
-    assert at(0) == 0 and at(blocks) == tiles
-    assert {at(b + 1) - at(b) for b in range(blocks)} <= {tq, tq + 1}
+@pytest.mark.parametrize("tiles,blocks,units", [(1, 1, 1), (257, 129, 1), (632, 211, 1), (2063, 768, 1), (1792, 224, 2),
+                                                (7, 1, 2), (6250, 1563, 1)])
+def test_tiles_and_blocks(tiles, blocks, units):
+    tq, tr = divmod(tiles, blocks * units)
+    at = lambda u: u * tq + min(u, tr)
+    assert at(0) == 0 and at(blocks * units) == tiles
+    assert {at(u + 1) - at(u) for u in range(blocks * units)} <= {tq, tq + 1}
     per, rem = divmod(blocks, 8)
     order = [(x * (per + 1) if x < rem else rem * (per + 1) + (x - rem) * per) + b // 8
              for b in range(blocks) for x in [b % 8]]
