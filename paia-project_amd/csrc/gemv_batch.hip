@@ -83,7 +83,7 @@ int launch_m1_b(BatchParams b, hipStream_t st)
 #define RV_ALL(F) RV_M(F, 1, 2, 8) RV_M(F, 2, 2, 4) RV_M(F, 1, 1, 8) RV_M(F, 2, 1, 4) RV_M(F, 1, 2, 16) \
                   RV_M(F, 2, 1, 16)
 // M = 5..8, BF16 and FP8 (INT4: 5, 6): BF16 has no decode (4 v_dot2 per 16 weight bytes and activation row), so 8 rows
-// stay within the VALU budget and the default pick streams them; FP8 and INT4 spend most of their VALU at M = 4 on the
+// stay within the VALU budget and the table's pick streams them; FP8 and INT4 spend most of their VALU at M = 4 on the
 // tall shapes, so only a measured entry (the tuned table) picks these for them, where they beat the matrix cores
 #define RV_M8(F, R, U, W) RV(F, R, U, W, 5) RV(F, R, U, W, 6) RV(F, R, U, W, 7) RV(F, R, U, W, 8)
 // INT4 at M = 5, 6 (seven and eight rows of staged x and lane sums do not fit the 16-wave launch's 128 VGPRs)
@@ -148,22 +148,23 @@ bool fits(const BatchVariant& v, int M)
     return v.X == 1 || batch_x_bytes(v.S, M, v.U) <= (v.X == 2 ? wide_lds() : kBatchLds);
 }
 
-// Default choice: a measured entry for the shape and M when the tuned table has one; otherwise a rule fitted to MI355X
-// sweeps of the Llama/Qwen projection shapes (FP8 and INT4). M = 1 takes the M = 1 GEMV when its staged x fits the LDS
-// (it beat the matrix-core kernel on every BASELINE shape: FP8 gate_up 18.9 µs against 22.7, INT4 asymmetric 12.2
-// against 16.5). M = 2..4 (BF16 2..8) take the row-streaming kernel when its x copies fit the LDS (pick_rows; BF16 at
-// M = 5..8 measured 9-37% faster than the matrix cores on every BASELINE shape where it fits); otherwise the
-// matrix-core kernel:
+// The table's choice, which paia_gemv_batch_pick_variant returns and a call left to the library runs where table_ahead
+// says so or the tile kernel refuses it (figures against the matrix-core kernel): a measured entry for the shape and M
+// when the tuned table has one; otherwise a rule fitted to MI355X sweeps of the Llama/Qwen projection shapes (FP8 and
+// INT4). M = 1 takes the M = 1 GEMV when its staged x fits the LDS (it beat the matrix-core kernel on every BASELINE
+// shape: FP8 gate_up 18.9 µs against 22.7, INT4 asymmetric 12.2 against 16.5). M = 2..4 (BF16 2..8) take the
+// row-streaming kernel when its x copies fit the LDS (pick_rows; BF16 at M = 5..8 measured 9-37% faster than the matrix
+// cores on every BASELINE shape where it fits); otherwise the matrix-core kernel:
 //   * split-K S: at least two splits (every shape streamed faster with two waves per tile than with one), then the
 //     fewest (<= 8, >= 2 k-blocks each) that give >= 1152 work units (tiles x splits, 4.5 per CU): qkv (384 tiles)
 //     measured best at S = 4, o/down (256 tiles) at S = 8, gate_up (1792 tiles) at S = 2;
 //   * x in LDS (X=0) unless the splits x rows make staging cost more than it saves (M*S >= 24 with S >= 4: each block
 //     would stage a third or more of its weight bytes again as x; measured at M = 3 on the tall-K down shapes, whose
-//     three x copies do not fit the row-streaming kernel: X=0 20.1 µs against 16.1 for X=1 at M = 4) or not even
-//     one chunk of U k-blocks fits;
-//   * one tile per wave; two when x comes with the weights and M >= 8, so the two tiles share each x load, provided
-//     the halved tile count still gives >= 1152 units within 8 splits (at 256 tiles it does not, and one tile per
-//     wave was faster there);
+//     three x copies do not fit the row-streaming kernel: X=0 20.1 µs against 16.1 for X=1 at M = 4) or not even one
+//     chunk of U k-blocks fits;
+//   * one tile per wave; two when x comes with the weights and M >= 8, so the two tiles share each x load, provided the
+//     halved tile count still gives >= 1152 units within 8 splits (at 256 tiles it does not, and one tile per wave was
+//     faster there);
 //   * x with the weights at M >= 8: four waves per block and at most four splits.
 constexpr int kPickUnits = 1152;
 
@@ -262,10 +263,12 @@ int pick(int kind, int M, int N, int K)
 // tile kernel takes the call where they do not (kRows) -- but for the one case whose entry is a matrix-core kernel
 // (kTable).
 //   * At most half a tile per CU, where a block per tile leaves half the CUs idle: BF16 to M = 7 (M = 4 4.30 / 5.25),
-//     at M = 8 even with rows of whole 128-byte lines, but split lines (next but one) are ahead from 1 MiB of weights
-//     on to 80 tiles, long rows from half of that to 112 (1168x2728 5.0 / 5.5, 592x3592 5.3 / 6.9, 350x9712 9.9 / 14.3,
-//     1376x7816 9.6 / 11.6; 160x1864 4.2 / 3.5, 1456x2984 6.4 / 5.9); FP8 to M = 4 (1000x3584 M = 2 3.22 / 3.86, M = 4
-//     3.76 / 4.12); INT4 M = 2 (3.48 / 4.2, 629x18048 8.3 / 10.6; M = 3 even) above K = 1536.
+//     at M = 8 even with rows of whole 128-byte lines (but for K = 3648..4096 to 80 tiles: 1040x4096 5.7 / 5.9); split
+//     lines (next but one) are ahead from 1 MiB of weights on to 80 tiles, long rows from half of that to 112
+//     (1168x2728 5.0 / 5.5, 592x3592 5.3 / 6.9, 350x9712 9.9 / 14.3, 1376x7816 9.6 / 11.6; 160x1864 4.2 / 3.5,
+//     1456x2984 6.4 / 5.9); FP8 to M = 4 (1000x3584 M = 2 3.22 / 3.86, M = 4 3.76 / 4.12); INT4 M = 2 (3.48 / 4.2,
+//     629x18048 8.3 / 10.6) above K = 1536, M = 3 at K = 3712..4096 above 32 tiles (1198x3968 4.5 / 5.0; elsewhere
+//     behind).
 //   * Ordinary K, up to 4 tiles per CU, BF16 to M = 3 (6144x4096 M = 2 9.60 / 10.86, M = 3 10.27 / 10.98, M = 4 even),
 //     FP8 M = 2 (6144x4096 6.51 / 7.10; M = 3 7.54 / 7.23), and the same at any N for K up to 2560 (BF16 33000x2048 M =
 //     2 21.5 / 22.4); BF16 rows beyond 16 KiB at one to two tiles per CU (5504x14336 M = 2 27.2 / 29.4, M = 5 29.2 /
@@ -282,8 +285,9 @@ int pick(int kind, int M, int N, int K)
 //     8-wave launch is 5 to 15% ahead), longer ones and FP8 above one (BF16 6760x16384 M = 5 49 / 75, FP8 12264x16256 M
 //     = 3 38.5 / 49.3); to M = 4 only up to 4 tiles per CU, as the block per tile beyond is even.
 //   * INT4 M = 2: up to a tile per CU and ordinary K (1455x1920 3.31 / 3.64), long rows on many tiles (30000x14336 43.0
-//     / 49.9, K = 6272..8192 on 1025..4096 tiles 0.88 to 0.98 of the tile kernel's, up to 6144 0.97 to 1.2), a great
-//     many of ordinary K (100000x4096 44.4 / 45.7, 70000x7168 53.3 / 55.2).
+//     / 49.9), rows that fill the row streaming's items of 2048 columns to nine tenths above 6 tiles per CU from K =
+//     3712 on, above 4 beyond K = 6144 (28672x4096 0.93 of the tile kernel's time, 2049..4096 tiles of K = 6144 0.87,
+//     8192 0.82, but 4224 1.1 to 1.2), a great many of ordinary K (100000x4096 44.4 / 45.7, 70000x7168 53.3 / 55.2).
 //   * FP8 split lines of at most 960 bytes at M = 5..8 above 18 tiles per CU: the matrix-core kernel (119226x528 M = 7
 //     18.4 / 22.8).
 enum Ahead { kTile, kRows, kTable };
@@ -293,9 +297,12 @@ Ahead table_ahead(int kind, int M, int N, int K)
     const int64_t nt = ((int64_t)N + kTileRows - 1) / kTileRows;
     auto rows = [](bool ahead) { return ahead ? kRows : kTile; };
     if (kind >= 2) {
+        const bool full = 10 * (int64_t)K >= 9 * (((int64_t)K + 2047) / 2048 * 2048);
+        if (M == 3) return rows(2 * nt <= cus && 8 * nt > cus && K >= 3712 && K <= 4096);
         if (M != 2) return kTile;
         if (2 * nt <= cus) return rows(K > 1536);
-        return rows((nt <= cus && K > 1536 && K <= 8192) || (nt > (K > 8192 ? 3 : 4) * cus && K > 6144) ||
+        if (K > 8192) return rows(nt > 3 * cus);
+        return rows((nt <= cus && K > 1536) || (full && K >= 3712 && nt > (K > 6144 ? 4 : 6) * cus) ||
                     (nt > 16 * cus && K >= 4096));
     }
     const bool bf16 = kind == 0, mid = K >= 2048 && K <= 8192;
@@ -303,7 +310,8 @@ Ahead table_ahead(int kind, int M, int N, int K)
     const bool split = row_bytes % 128 != 0;
     if (2 * nt <= cus) {
         if (!bf16 || M < 8) return rows(M <= (bf16 ? 7 : 4));
-        if (!split || M > 8) return kTile;
+        if (M > 8) return kTile;
+        if (!split) return rows(K > 3584 && K <= 4096 && 16 * nt <= 5 * cus);
         if (K < 4096) return rows(K >= 1408 && nt * K >= 32768 && 16 * nt <= 5 * cus);
         return rows((K > 8192 || nt * K >= 16384) && 16 * nt <= 7 * cus);
     }

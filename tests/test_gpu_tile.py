@@ -249,7 +249,10 @@ ROUTES = [("bf16", 8, 592, 3592, True), ("bf16", 8, 350, 9712, True), ("bf16", 8
           ("fp8", 3, 36392, 2160, False), ("fp8", 3, 12264, 16256, True), ("fp8", 5, 12264, 16256, False),
           ("fp8", 7, 74000, 528, True), ("fp8", 7, 73000, 528, False), ("fp8", 9, 74000, 528, False),
           ("int4", 2, 629, 18048, True), ("int4zp", 2, 629, 18048, True), ("int4", 2, 17000, 7552, True),
-          ("int4zp", 2, 17000, 6016, False),
+          ("int4zp", 2, 17000, 6016, False), ("int4zp", 2, 25000, 6016, True),
+          ("int4zp", 2, 25000, 5504, False),
+          ("int4", 2, 28672, 4096, True), ("int4", 2, 20000, 4096, False), ("int4", 3, 1400, 3968, True),
+          ("bf16", 8, 1024, 4096, True),
           # six tiles per wave: metadata beyond the LDS above K = 37376
           ("int4", 16, 24576, 38400, True), ("int4zp", 16, 24576, 37376, False)]
 
