@@ -264,7 +264,7 @@ int pick(int kind, int M, int N, int K)
 // (kTable).
 //   * At most half a tile per CU, where a block per tile leaves half the CUs idle: BF16 to M = 7 (M = 4 4.30 / 5.25),
 //     at M = 8 even with rows of whole 128-byte lines (but for K = 3648..4096 to 80 tiles: 1040x4096 5.7 / 5.9); split
-//     lines (next but one) are ahead from 1 MiB of weights on to 80 tiles, long rows from half of that to 112
+//     lines (next but one) are ahead from 1 MiB of weights on to 80 tiles, from K = 4608 on from 3/4 of that to 112
 //     (1168x2728 5.0 / 5.5, 592x3592 5.3 / 6.9, 350x9712 9.9 / 14.3, 1376x7816 9.6 / 11.6; 160x1864 4.2 / 3.5,
 //     1456x2984 6.4 / 5.9); FP8 to M = 4 (1000x3584 M = 2 3.22 / 3.86, M = 4 3.76 / 4.12); INT4 M = 2 (3.48 / 4.2,
 //     629x18048 8.3 / 10.6) above K = 1536, M = 3 at K = 3712..4096 above 32 tiles (1198x3968 4.5 / 5.0; elsewhere
@@ -312,8 +312,8 @@ Ahead table_ahead(int kind, int M, int N, int K)
         if (!bf16 || M < 8) return rows(M <= (bf16 ? 7 : 4));
         if (M > 8) return kTile;
         if (!split) return rows(K > 3584 && K <= 4096 && 16 * nt <= 5 * cus);
-        if (K < 4096) return rows(K >= 1408 && nt * K >= 32768 && 16 * nt <= 5 * cus);
-        return rows((K > 8192 || nt * K >= 16384) && 16 * nt <= 7 * cus);
+        if (K < 4608) return rows(K >= 1600 && nt * K >= 32768 && 16 * nt <= 5 * cus);
+        return rows((K > 8192 || nt * K >= 24576) && 16 * nt <= 7 * cus);
     }
     if (split) {
         if (K <= 8192 && M <= (bf16 ? 4 : 2)) return kRows;
