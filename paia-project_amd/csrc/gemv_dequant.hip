@@ -12,11 +12,14 @@
 
 namespace paia {
 
-// Bound by the fp32 stores (4 bytes a weight against 0.5 to 1 read): a lane takes 4 neighbouring weights, so a wave's store
-// is 1 KiB in a row and every line leaves whole. With 16 or 32 weights a lane, four or eight stores each touched a quarter
-// or an eighth of 64 lines (28672x4096: FP8 170 us, INT4 162, INT4ZP 156; now 83, 76 and 75). The stores are non-temporal
-// (each byte is written once and nothing here reads it back). A block takes 4096 columns of a row (1024 in calls of few
-// weights, where four steps a lane and a quarter of the blocks cost 0.3 to 1.3 us), or for short rows as many whole rows as fit; `mul` = ceil(2^32 / K) then divides a weight's index in the block by K (index * K < 2^32).
+// Bound by the fp32 stores (4 bytes a weight against 0.5 to 1 read): a lane takes 4 neighbouring weights, so a wave's
+// store is 1 KiB in a row and every line leaves whole. With 16 or 32 weights a lane, four or eight stores each touched a
+// quarter or an eighth of 64 lines. 28672x4096 launched again and again (the codes then come from the Infinity Cache):
+// FP8 169 us, INT4 168, INT4ZP 156; now 83, 74 and 72. In turn with other kernels, codes from HBM: 160, 163 and 159; now
+// 96, 114 and 116. The stores are non-temporal (each byte is written once and nothing here reads it back). A block takes
+// 4096 columns of a row (1024 in calls of few weights, where four steps a lane and a quarter of the blocks cost 0.3 to
+// 1.3 us), or for short rows as many whole rows as fit; `mul` = ceil(2^32 / K) then divides a weight's index in the
+// block by K (index * K < 2^32).
 constexpr int kDqThreads = 256;
 constexpr int dq_block(int steps) { return kDqThreads * 4 * steps; }   // weights per block
 

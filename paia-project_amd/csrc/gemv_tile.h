@@ -114,7 +114,9 @@ __device__ __forceinline__ uint32_t i4x2_to_bf16x2(uint32_t w, float scale)
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, HI));
 }
 
-// P tiles per unit, S waves sharing them along K (W / S units per block), D stages in flight per wave, MT activation
+// P tiles per unit, S waves sharing them along K (W / S units per block; every launch has one, S = W, but the schedule the
+// compiler finds with the single unit written in was 0.5 to 3% slower: INT4ZP 14336x4096 M = 8 10.04 -> 10.09 us,
+// 58559x4608 36.0 -> 37.2), D stages in flight per wave, MT activation
 // rows staged (4, 8 or 16 >= M), AUX cache policy of the weight loads, IL: a unit's waves take the stages in turn
 // (neighbouring waves read neighbouring bytes of a row) rather than a contiguous range each.
 // RING (BF16, FP8; not IL): for rows that are no multiple of 128 bytes, where a stage's 128 bytes of a row lie in two lines

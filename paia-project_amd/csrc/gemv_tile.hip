@@ -12,9 +12,10 @@ namespace {
 //   * W waves split the K of P tiles. BF16 and FP8 run best as 4-wave blocks, several to a CU, so that one block's start and
 //     end lie under another's stream (FP8 28672x4096 M = 16 20.6 with 4 waves, 21.5 with 8; 10112x4096 10.0 / 11.1; BF16
 //     33000x2048 22.6 / 26.0); but a BF16 row beyond 8 KiB keeps one 4-wave block per CU from having enough in flight
-//     (9216x8192 M = 8 34.9 with 4 waves, 26.4 with 8; 4096x14336 M = 4 21.1 / 20.5). INT4 spends as long on decoding
-//     a stage as on reading it and wants more waves on it (4096x14336 M = 4 9.9 with 8 waves, 12.4 with 4), except for short rows, which leave 8 waves a stage or none each
-//     (100000x512 M = 4 9.4 with 4, 12.1 with 8; one tile per CU: 300x1024 2.86 / 2.95, but 2048x2048 3.72 / 3.53).
+//     (9216x8192 M = 8 34.9 with 4 waves, 26.4 with 8; 4096x14336 M = 4 21.1 / 20.5). INT4 keeps its matrix cores and VALU
+//     waiting between a stage's loads and its decode and wants more waves (4096x14336 M = 4 9.9 with 8 waves, 12.4 with
+//     4), except for short rows, which leave 8 waves a stage or none each (100000x512 M = 4 9.4 with 4, 12.1 with 8; one
+//     tile per CU: 300x1024 2.86 / 2.95, but 2048x2048 3.72 / 3.53).
 //   * D stages in flight. One tile per wave: the stages of a K = 4096 row at once (FP8 4096x4096 M = 4 5.06 with four, 5.6
 //     with two), two for FP8 at 16 activation rows (registers) and for INT4 up to 8 stages per wave (4096x4096 4.97 /
 //     5.16 with four; 4096x14336 10.98 / 9.49). More tiles need fewer, and a second stage soon costs more registers than it

@@ -18,9 +18,11 @@
 //   threads for K <= 32768; beyond, the row is read twice). With rows read twice, the second time from L2, 4096x14336 took
 //   88 us (512 KiB of rows per CU in flight is more than its share of L2) and 28672x4096 121; now 47 and 89 (6.6 TB/s).
 //   The loads are non-temporal: a row's bytes are used once (plain: 56 and 105 us).
-//   INT4: a group is 16 lanes of 8 weights, so its maximum takes four DPP steps, its scale one conversion per lane and its
-//   codes leave as 4 bytes a lane; a wave holds 8 groups. With a group per wave (2 weights and 1 byte a lane) 28672x4096 took
-//   141 us, asymmetric 183; now 96 both (5.5 TB/s). Plain loads: a lane's two 16-byte loads share lines (non-temporal 99).
+//   INT4: a group is 16 lanes of 8 weights, so its maximum takes four DPP steps, its scale one conversion per lane and
+//   its codes leave as 4 bytes a lane; a wave holds 8 groups. With a group per wave (2 weights and 1 byte a lane)
+//   28672x4096 took 147 us, asymmetric 195; now 96 both (5.5 TB/s; in turn with other kernels 149 and 200, now 102 and
+//   96). Plain loads: a lane's two 16-byte loads share lines (non-temporal 99).
+//   Calls of few weights take fewer of them a lane (kFewWeights).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
